@@ -45,7 +45,7 @@ def _run(cmd):
 
 
 HIP_SOURCES = ["tbe_nbit.hip", "tbe_kern_int4.hip", "tbe_kern_int8.hip", "tbe_kern_int2.hip", "tbe_kern_fp8.hip",
-               "tbe_kern_fp16.hip", "tbe_kern_fp32.hip", "pooled_ops.hip", "sparse_ops.hip"]
+               "tbe_kern_fp16.hip", "tbe_kern_fp32.hip", "tbe_kern_any.hip", "pooled_ops.hip", "sparse_ops.hip"]
 OBJ_DIR = os.path.join(PKG_DIR, "_build")
 
 

@@ -1612,6 +1612,12 @@ __global__ __launch_bounds__(kBlock) void pooled_wide_kernel(KParams p) {
 
 using KernelFn = void (*)(KParams);
 
+// tbe_kern_any.hip: the one kernel for tables of every type and width (split: a
+// work-group per item, else a wave), and the column tiles it cuts a row into that
+// the planner counted as `col_tiles` tiles of 64 words.
+KernelFn any_kernel(bool index64, bool weighted, bool split);
+int any_col_tiles(int weight_ty, int col_tiles);
+
 template <int WT, int LG, int VW>
 KernelFn fast_kernel_vw(bool index64, bool weighted) {
   if (index64)

@@ -263,6 +263,30 @@ KernelFn pooled_kernel_for(const TbePlanGroup& g, bool index64, bool weighted, b
   }
 }
 
+// Calls of several table groups with at most this many bags take the one kernel for
+// every type and width (tbe_kern_any.hip) instead of a launch per group: 15 launches of
+// 5 us kernels cost ~95 us whatever the batch.  64 mixed tables (weighted mean, 32 rows
+// a bag): 2 k bags 93 -> 7 us, 32 k bags 95 -> 33, 131 k bags 182 -> 132, 262 k bags
+// 286 -> 266; past it the specialised kernels' pipeline over bags wins (524 k bags 461
+// against 516 us).
+constexpr int64_t kAnyMaxBags = int64_t(1) << 18;
+
+bool use_any_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan) {
+  // the flags that choose a kernel per group keep doing so
+  if (a->flags & (TBE_FLAG_NO_STREAM | TBE_FLAG_FORCE_STREAM | TBE_FLAG_NARROW_WORDS)) return false;
+  if (plan.num_groups < 2 || a->num_indices > 0x7FFFFFFF || static_cast<int64_t>(a->T) * a->B > kAnyMaxBags)
+    return false;
+  for (int gi = 0; gi < plan.num_groups; ++gi)  // 32-bit row offsets only
+    if (!plan.groups[gi].offset32) return false;
+  return true;
+}
+
+// Four waves per bag instead of one when bags are long and too few to fill the GPU
+// (items: bags x column tiles).  The line lies where both run alike: 512 bags of 32 rows
+// 6.6 (one wave) against 5.8 us, 2048 bags of 32 rows 8.8 against 11.0, of 64 rows 14.5
+// against 14.4, of 100 rows 20.2 against 18.0 (16 float tables of 64-512 columns).
+bool any_split(int64_t items, int64_t rows_per_bag) { return rows_per_bag >= 32 && items <= 32 * rows_per_bag; }
+
 // Blocks of `fn` the whole GPU keeps resident at once (cached per device and kernel).
 int resident_blocks(KernelFn fn) {
   static std::mutex mu;
@@ -578,6 +602,20 @@ int tbe_nbit_forward(const TbeNbitArgs* a, void* hip_stream) {
   const bool weighted = a->indice_weights != nullptr;
   // the per-group kernels keep index positions in 32 bits
   const bool wide = a->num_indices > 0x7FFFFFFF;
+  if (use_any_kernel(a, plan)) {
+    int tiles = 1;
+    for (int gi = 0; gi < plan.num_groups; ++gi)
+      tiles = std::max(tiles, any_col_tiles(plan.groups[gi].weight_ty, plan.groups[gi].col_tiles));
+    const int64_t items = nbags * tiles;
+    const bool split = any_split(items, a->num_indices / nbags);
+    p.col_tiles = tiles;
+    p.div_tiles = make_fastdiv(static_cast<uint32_t>(tiles));
+    p.num_items = static_cast<int32_t>(items);
+    const hipError_t err = launch(any_kernel(p.index64 != 0, weighted, split), p,
+                                  split ? items : (items + kWavesPerBlock - 1) / kWavesPerBlock, false, s);
+    if (err != hipSuccess) return fail(TBE_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+    return TBE_OK;
+  }
   // several groups: launch them on the group streams, between a fork and a join
   GroupStreams* gs = (plan.num_groups > 1 && !(a->flags & TBE_FLAG_SERIAL_GROUPS)) ? group_streams(s) : nullptr;
   std::unique_lock<std::mutex> gs_lock;

@@ -1,0 +1,36 @@
+"""The one-launch pooled kernel (calls of several table groups): rows at the edges of its
+words per lane and column tiles, bags at the edges of its row steps, both waves per bag,
+against the CPU oracle with the tolerance of tests/_parity.py."""
+import pytest
+import torch
+
+from test_gpu_parity import BF16, FP8, FP16, FP32, INT2, INT4, INT8, _check_module
+
+pytestmark = pytest.mark.gpu
+
+PER_WORD = {FP32: 1, FP16: 2, BF16: 2, FP8: 4, INT8: 4, INT4: 8, INT2: 16}
+# payload words: 1-4 lanes, a full tile and one past it, two and four words per lane with
+# a cut last lane, more than one tile of four
+WORDS = (1, 3, 5, 63, 64, 65, 127, 129, 131, 257)
+
+
+@pytest.mark.parametrize("lengths", ["short", "long"])
+@pytest.mark.parametrize("weighted,index,pm,out", [(False, torch.int32, 0, FP32), (True, torch.int64, 1, FP32),
+                                                   (False, torch.int64, 1, FP16), (True, torch.int32, 0, BF16)])
+@pytest.mark.parametrize("ty", sorted(PER_WORD))
+def test_any_kernel_edges(pkg, oracle, gpu, ty, weighted, index, pm, out, lengths):
+    specs = [(40 + 7 * i, w * PER_WORD[ty], pkg.SparseType(ty)) for i, w in enumerate(WORDS)]
+    m = pkg.IntNBitTableBatchedEmbeddingBagsCodegen(specs, device=gpu, pooling_mode=pm, output_dtype=out,
+                                                    indices_dtype=index)
+    m.fill_random_weights(11)
+    # "long" bags average over 32 rows, so four waves share one; "short" ones take a wave
+    lens = [0, 1, 2, 7, 8, 9, 16, 33] if lengths == "short" else [0, 1, 3, 31, 64, 65, 129, 200]
+    g = torch.Generator(device=gpu)
+    g.manual_seed(5)
+    L = torch.tensor([lens[(i + t) % len(lens)] for t in range(len(specs)) for i in range(len(lens))], device=gpu)
+    per = len(lens)
+    idx = torch.cat([torch.randint(-1, E + 1, (int(L[t * per:(t + 1) * per].sum()),), device=gpu, generator=g)
+                     for t, (E, _, _) in enumerate(specs)]).to(index)  # -1 and E: skipped rows
+    off = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), L.cumsum(0)]).to(index)
+    psw = torch.rand(idx.numel(), device=gpu, generator=g) if weighted else None
+    _check_module(oracle, m, idx, off, psw, f"any ty={ty} {lengths}")
