@@ -220,7 +220,10 @@ __global__ __launch_bounds__(kBlock) void pooled_any_kernel(KParams p) {
     case TBE_TY_INT4: any_table<TBE_TY_INT4, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;
     case TBE_TY_INT8: any_table<TBE_TY_INT8, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;
     case TBE_TY_INT2: any_table<TBE_TY_INT2, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;
-    case TBE_TY_FP8:  any_table<TBE_TY_FP8,  WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;
+    case TBE_TY_FP8:
+      if (p.fp8.h16_ok) any_table<TBE_TY_FP8, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh);
+      else any_table<kTyFp8Wide, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh);
+      break;
     case TBE_TY_FP16: any_table<TBE_TY_FP16, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;
     case TBE_TY_BF16: any_table<TBE_TY_BF16, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;
     case TBE_TY_FP32: any_table<TBE_TY_FP32, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;

@@ -86,9 +86,10 @@ struct Fp8Consts {
   uint32_t mant_bits;  // 7 - exponent_bits
   float mult;          // 2^(127 - bias) (C:131)
   float sub_scale;     // 2^(1 - bias - mant_bits): value of one unit of a subnormal body
-  uint32_t h16_shift;  // exponent_bits + 3: body bits -> fp16 exponent/mantissa field
+  uint32_t h16_shr;    // 5 - exponent_bits in both halves: top of a half -> fp16 exponent/mantissa field
+  uint32_t h16_mask;   // sign and body bits of both halves after that shift
   float h16_scale;     // 2^(15 - bias): fp16 reading of the placed body -> code value
-  int32_t h16_ok;      // exponent_bits <= 4: every body fits a finite fp16
+  int32_t h16_ok;      // exponent_bits <= 4: every body fits a finite fp16 (else the kTyFp8Wide kernels)
   float one;           // 1.0f (see accum_row)
 };
 
@@ -195,11 +196,17 @@ __device__ __forceinline__ uint32_t load_word(const uint8_t* p) {
 
 // ---------------------------------------------------------------- element decode
 
+// FP8 rows whose codes do not all fit a finite fp16 (5 or more exponent bits).  A kernel
+// of its own: chosen per element by a uniform branch, the two decodes cost the FP8 kernels
+// three jumps and their register moves per payload word.
+constexpr int kTyFp8Wide = 7;
+
 template <int WT> struct Traits;
 template <> struct Traits<TBE_TY_FP32> { static constexpr int kEpd = 1;  static constexpr bool kHdr = false; };
 template <> struct Traits<TBE_TY_FP16> { static constexpr int kEpd = 2;  static constexpr bool kHdr = false; };
 template <> struct Traits<TBE_TY_BF16> { static constexpr int kEpd = 2;  static constexpr bool kHdr = false; };
 template <> struct Traits<TBE_TY_FP8>  { static constexpr int kEpd = 4;  static constexpr bool kHdr = false; };
+template <> struct Traits<kTyFp8Wide>  { static constexpr int kEpd = 4;  static constexpr bool kHdr = false; };
 template <> struct Traits<TBE_TY_INT8> { static constexpr int kEpd = 4;  static constexpr bool kHdr = true; };
 template <> struct Traits<TBE_TY_INT4> { static constexpr int kEpd = 8;  static constexpr bool kHdr = true; };
 template <> struct Traits<TBE_TY_INT2> { static constexpr int kEpd = 16; static constexpr bool kHdr = true; };
@@ -234,7 +241,7 @@ __device__ __forceinline__ void decode(uint32_t d, float (&v)[Traits<WT>::kEpd],
   } else if constexpr (WT == TBE_TY_BF16) {
     v[0] = __uint_as_float(d << 16);
     v[1] = __uint_as_float(d & 0xFFFF0000u);
-  } else if constexpr (WT == TBE_TY_FP8) {
+  } else if constexpr (WT == TBE_TY_FP8 || WT == kTyFp8Wide) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = fp8_decode((d >> (8 * e)) & 0xFFu, c);
   } else {
@@ -265,6 +272,14 @@ __device__ __forceinline__ float acc_post_scale(int e) {
     return __int_as_float((127 + 24 - 2 * jp) << 23);
   }
   return WT == TBE_TY_INT8 ? 16777216.0f : 1.0f;
+}
+
+typedef int16_t short2_t __attribute__((ext_vector_type(2)));
+
+// Two FP8 codes, each in the upper byte of a half, as the fp16 values code * 2^(bias-15).
+__device__ __forceinline__ uint32_t fp8_halves(uint32_t x, const Fp8Consts& c) {
+  const short2_t s = __builtin_bit_cast(short2_t, x) >> __builtin_bit_cast(short2_t, c.h16_shr);
+  return __builtin_bit_cast(uint32_t, s) & c.h16_mask;
 }
 
 // Add one row's contribution: acc[e] += w * value[e] (value = scale*q + bias for INT
@@ -325,24 +340,17 @@ __device__ __forceinline__ void accum_row(float (&acc)[Traits<WT>::kEpd], float&
       acc[1] += h16hi(d);
     }
   } else if constexpr (WT == TBE_TY_FP8) {
-    if (c.h16_ok) {
-      // place each 7-bit body into an fp16 exponent/mantissa field, sign to bit 15:
-      // fp16 value * 2^(15-bias) is the code's value (subnormal codes included)
-      const float m = WEIGHTED ? c.h16_scale * w : c.h16_scale;
-      const uint32_t x0 = d & 0x00FF00FFu, x1 = (d >> 8) & 0x00FF00FFu;
-      const uint32_t p0 = ((x0 & 0x007F007Fu) << c.h16_shift) | ((x0 & 0x00800080u) << 8);
-      const uint32_t p1 = ((x1 & 0x007F007Fu) << c.h16_shift) | ((x1 & 0x00800080u) << 8);
-      acc[0] = fmaf(h16lo(p0), m, acc[0]);
-      acc[2] = fmaf(h16hi(p0), m, acc[2]);
-      acc[1] = fmaf(h16lo(p1), m, acc[1]);
-      acc[3] = fmaf(h16hi(p1), m, acc[3]);
-    } else {
-      float v[E];
-      decode<WT>(d, v, c);
-#pragma unroll
-      for (int e = 0; e < E; ++e) acc[e] = WEIGHTED ? fmaf(v[e], w, acc[e]) : acc[e] + v[e];
-    }
-  } else {  // FP32, BF16
+    // each byte goes to the top of a half, an arithmetic shift brings its 7-bit body into
+    // the fp16 exponent/mantissa field and keeps the sign in bit 15, the mask clears the
+    // sign's copies: the fp16 value * 2^(15-bias) is the code's value (subnormal codes too)
+    const float m = WEIGHTED ? c.h16_scale * w : c.h16_scale;
+    const uint32_t p0 = fp8_halves(__builtin_amdgcn_perm(d, d, 0x010C000Cu), c);  // elements 0 and 1
+    const uint32_t p1 = fp8_halves(__builtin_amdgcn_perm(d, d, 0x030C020Cu), c);  // elements 2 and 3
+    acc[0] = fmaf(h16lo(p0), m, acc[0]);
+    acc[1] = fmaf(h16hi(p0), m, acc[1]);
+    acc[2] = fmaf(h16lo(p1), m, acc[2]);
+    acc[3] = fmaf(h16hi(p1), m, acc[3]);
+  } else {  // FP32, BF16, FP8 of 5 or more exponent bits
     float v[E];
     decode<WT>(d, v, c);
 #pragma unroll
@@ -1601,7 +1609,7 @@ __global__ __launch_bounds__(kBlock) void pooled_wide_kernel(KParams p) {
       case TBE_TY_INT4: pool_bag_wide<TBE_TY_INT4, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_INT8: pool_bag_wide<TBE_TY_INT8, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_INT2: pool_bag_wide<TBE_TY_INT2, WEIGHTED>(p, td, start, L, ct, b); break;
-      case TBE_TY_FP8:  pool_bag_wide<TBE_TY_FP8,  WEIGHTED>(p, td, start, L, ct, b); break;
+      case TBE_TY_FP8:  pool_bag_wide<kTyFp8Wide,  WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_FP16: pool_bag_wide<TBE_TY_FP16, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_BF16: pool_bag_wide<TBE_TY_BF16, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_FP32: pool_bag_wide<TBE_TY_FP32, WEIGHTED>(p, td, start, L, ct, b); break;

@@ -34,6 +34,9 @@ extern template KernelFn fast_kernel_lg<TBE_TY_FP8>(int, bool, bool, bool);
 extern template KernelFn fast_kernel_a64_lg<TBE_TY_FP8>(int, bool, bool);
 extern template KernelFn stream_kernel_lg<TBE_TY_FP8>(int, bool, bool);
 extern template KernelFn nobag_kernel_lg<TBE_TY_FP8>(int, bool, bool);
+extern template KernelFn fast_kernel_lg<kTyFp8Wide>(int, bool, bool, bool);
+extern template KernelFn fast_kernel_a64_lg<kTyFp8Wide>(int, bool, bool);
+extern template KernelFn stream_kernel_lg<kTyFp8Wide>(int, bool, bool);
 extern template KernelFn fast_kernel_lg<TBE_TY_INT8>(int, bool, bool, bool);
 extern template KernelFn fast_kernel_a64_lg<TBE_TY_INT8>(int, bool, bool);
 extern template KernelFn stream_kernel_lg<TBE_TY_INT8>(int, bool, bool);
@@ -162,7 +165,10 @@ Fp8Consts make_fp8(int bits, int bias) {
   const uint32_t mult_bits = static_cast<uint32_t>(254 - bias) << 23;
   memcpy(&c.mult, &mult_bits, 4);
   c.sub_scale = ldexpf(1.0f, 1 - bias - (7 - bits));
-  c.h16_shift = static_cast<uint32_t>(bits + 3);
+  const uint32_t shr = static_cast<uint32_t>(std::max(0, 5 - bits));
+  const uint32_t half = 0x8000u | ((0x7F00u >> shr) & 0x7FFFu);
+  c.h16_shr = shr | (shr << 16);
+  c.h16_mask = half | (half << 16);
   c.h16_scale = ldexpf(1.0f, 15 - bias);
   c.h16_ok = bits <= 4;
   return c;
@@ -178,13 +184,19 @@ FastDiv make_fastdiv(uint32_t d) {
   return f;
 }
 
+// The type whose kernels pool a group: FP8 codes that do not fit fp16 have their own.
+int kernel_ty(const TbePlanGroup& g, const Fp8Consts& fp8) {
+  return g.weight_ty == TBE_TY_FP8 && !fp8.h16_ok ? kTyFp8Wide : g.weight_ty;
+}
+
 // Row-stream kernel of a group (rows of >= 16 lanes, 32-bit table offsets).
-KernelFn stream_kernel_group(const TbePlanGroup& g, bool index64, bool weighted) {
-  switch (g.weight_ty) {
+KernelFn stream_kernel_group(const TbePlanGroup& g, bool index64, bool weighted, const Fp8Consts& fp8) {
+  switch (kernel_ty(g, fp8)) {
     case TBE_TY_FP32: return stream_kernel_lg<TBE_TY_FP32>(g.log2_lanes, index64, weighted);
     case TBE_TY_FP16: return stream_kernel_lg<TBE_TY_FP16>(g.log2_lanes, index64, weighted);
     case TBE_TY_BF16: return stream_kernel_lg<TBE_TY_BF16>(g.log2_lanes, index64, weighted);
     case TBE_TY_FP8:  return stream_kernel_lg<TBE_TY_FP8>(g.log2_lanes, index64, weighted);
+    case kTyFp8Wide:  return stream_kernel_lg<kTyFp8Wide>(g.log2_lanes, index64, weighted);
     case TBE_TY_INT8: return stream_kernel_lg<TBE_TY_INT8>(g.log2_lanes, index64, weighted);
     case TBE_TY_INT4: return stream_kernel_lg<TBE_TY_INT4>(g.log2_lanes, index64, weighted);
     default:          return stream_kernel_lg<TBE_TY_INT2>(g.log2_lanes, index64, weighted);
@@ -239,24 +251,27 @@ KernelFn nobag_kernel_group(const TbePlanGroup& g, bool index64) {
   }
 }
 
-KernelFn pooled_kernel_for(const TbePlanGroup& g, bool index64, bool weighted, bool wide, bool wide_words) {
+KernelFn pooled_kernel_for(const TbePlanGroup& g, bool index64, bool weighted, bool wide, bool wide_words,
+                           const Fp8Consts& fp8) {
   if (wide || g.weight_ty < 0) return weighted ? pooled_wide_kernel<true> : pooled_wide_kernel<false>;
   if (!g.offset32) {  // past 32-bit byte offsets: 64-bit row addresses
-    switch (g.weight_ty) {
+    switch (kernel_ty(g, fp8)) {
       case TBE_TY_FP32: return fast_kernel_a64_lg<TBE_TY_FP32>(g.log2_lanes, index64, weighted);
       case TBE_TY_FP16: return fast_kernel_a64_lg<TBE_TY_FP16>(g.log2_lanes, index64, weighted);
       case TBE_TY_BF16: return fast_kernel_a64_lg<TBE_TY_BF16>(g.log2_lanes, index64, weighted);
       case TBE_TY_FP8:  return fast_kernel_a64_lg<TBE_TY_FP8>(g.log2_lanes, index64, weighted);
+      case kTyFp8Wide:  return fast_kernel_a64_lg<kTyFp8Wide>(g.log2_lanes, index64, weighted);
       case TBE_TY_INT8: return fast_kernel_a64_lg<TBE_TY_INT8>(g.log2_lanes, index64, weighted);
       case TBE_TY_INT4: return fast_kernel_a64_lg<TBE_TY_INT4>(g.log2_lanes, index64, weighted);
       default:          return fast_kernel_a64_lg<TBE_TY_INT2>(g.log2_lanes, index64, weighted);
     }
   }
-  switch (g.weight_ty) {
+  switch (kernel_ty(g, fp8)) {
     case TBE_TY_FP32: return fast_kernel_lg<TBE_TY_FP32>(g.log2_lanes, index64, weighted, wide_words);
     case TBE_TY_FP16: return fast_kernel_lg<TBE_TY_FP16>(g.log2_lanes, index64, weighted, wide_words);
     case TBE_TY_BF16: return fast_kernel_lg<TBE_TY_BF16>(g.log2_lanes, index64, weighted, wide_words);
     case TBE_TY_FP8:  return fast_kernel_lg<TBE_TY_FP8>(g.log2_lanes, index64, weighted, wide_words);
+    case kTyFp8Wide:  return fast_kernel_lg<kTyFp8Wide>(g.log2_lanes, index64, weighted, wide_words);
     case TBE_TY_INT8: return fast_kernel_lg<TBE_TY_INT8>(g.log2_lanes, index64, weighted, wide_words);
     case TBE_TY_INT4: return fast_kernel_lg<TBE_TY_INT4>(g.log2_lanes, index64, weighted, wide_words);
     default:          return fast_kernel_lg<TBE_TY_INT2>(g.log2_lanes, index64, weighted, wide_words);
@@ -668,7 +683,7 @@ int tbe_nbit_forward(const TbeNbitArgs* a, void* hip_stream) {
                             ((a->flags & TBE_FLAG_FORCE_STREAM) || group_bags >= kStreamMinBags);
     if (!wide && use_stream) {
       // one wave per (table, range of bags, column tile), no persistence
-      const KernelFn fn = stream_kernel_group(g, p.index64 != 0, weighted);
+      const KernelFn fn = stream_kernel_group(g, p.index64 != 0, weighted, p.fp8);
       const double rows_per_bag = static_cast<double>(a->num_indices) / static_cast<double>(std::max<int64_t>(1, a->T * a->B));
       p.bags_per_wave = stream_bags_per_wave(group_bags,
                                              static_cast<int64_t>(resident_blocks(fn)) * kWavesPerBlock, rows_per_bag);
@@ -684,7 +699,7 @@ int tbe_nbit_forward(const TbeNbitArgs* a, void* hip_stream) {
       p.xcd = (p.xcd & 1) | (plan.num_groups == 1 ? 2 : 0);
       // two words per lane when every table of the group has an even word count
       const bool wide_words = g.stream && !(a->flags & TBE_FLAG_NARROW_WORDS);
-      err = launch(pooled_kernel_for(g, p.index64 != 0, weighted, wide, wide_words), p,
+      err = launch(pooled_kernel_for(g, p.index64 != 0, weighted, wide, wide_words, p.fp8), p,
                    (items + kWavesPerBlock - 1) / kWavesPerBlock, true, gstream);
     }
   }

@@ -18,10 +18,11 @@ WORDS = (1, 3, 5, 63, 64, 65, 127, 129, 131, 257)
 @pytest.mark.parametrize("weighted,index,pm,out", [(False, torch.int32, 0, FP32), (True, torch.int64, 1, FP32),
                                                    (False, torch.int64, 1, FP16), (True, torch.int32, 0, BF16)])
 @pytest.mark.parametrize("ty", sorted(PER_WORD))
-def test_any_kernel_edges(pkg, oracle, gpu, ty, weighted, index, pm, out, lengths):
+def test_any_kernel_edges(pkg, oracle, gpu, ty, weighted, index, pm, out, lengths, fp8=(4, 7)):
     specs = [(40 + 7 * i, w * PER_WORD[ty], pkg.SparseType(ty)) for i, w in enumerate(WORDS)]
     m = pkg.IntNBitTableBatchedEmbeddingBagsCodegen(specs, device=gpu, pooling_mode=pm, output_dtype=out,
-                                                    indices_dtype=index)
+                                                    indices_dtype=index, fp8_exponent_bits=fp8[0],
+                                                    fp8_exponent_bias=fp8[1])
     m.fill_random_weights(11)
     # "long" bags average over 32 rows, so four waves share one; "short" ones take a wave
     lens = [0, 1, 2, 7, 8, 9, 16, 33] if lengths == "short" else [0, 1, 3, 31, 64, 65, 129, 200]
@@ -34,3 +35,10 @@ def test_any_kernel_edges(pkg, oracle, gpu, ty, weighted, index, pm, out, length
     off = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), L.cumsum(0)]).to(index)
     psw = torch.rand(idx.numel(), device=gpu, generator=g) if weighted else None
     _check_module(oracle, m, idx, off, psw, f"any ty={ty} {lengths}")
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("bits,bias", [(1, 3), (2, 5), (3, 0), (5, 15), (7, 60)])
+def test_any_kernel_fp8_formats(pkg, oracle, gpu, bits, bias, weighted):
+    # up to 4 exponent bits codes are read as shifted fp16 halves, above through fp32
+    test_any_kernel_edges(pkg, oracle, gpu, FP8, weighted, torch.int32, 0, FP32, "short", fp8=(bits, bias))
