@@ -200,8 +200,9 @@ __global__ __launch_bounds__(kBlock) void pooled_any_kernel(KParams p) {
     k = fast_div(item, p.div_tiles);
     ct = static_cast<int>(item - k * static_cast<uint32_t>(p.col_tiles));
   }
-  const int32_t t = uniform(static_cast<int>(fast_div(k, p.div_B)));
-  const int64_t b = static_cast<int64_t>(k - static_cast<uint32_t>(t) * static_cast<uint32_t>(p.B));
+  const int32_t gt = uniform(static_cast<int>(fast_div(k, p.div_B)));
+  const int64_t b = static_cast<int64_t>(k - static_cast<uint32_t>(gt) * static_cast<uint32_t>(p.B));
+  const int32_t t = p.order ? load_uniform(p.order + p.group_first + gt) : gt;  // one group, or every table
   const TbeTableDesc td = load_desc(p.tables + t);
   const int64_t bag = static_cast<int64_t>(t) * p.B + b;
   // clamp to the index array so malformed offsets can never read out of bounds

@@ -203,9 +203,11 @@ KernelFn stream_kernel_group(const TbePlanGroup& g, bool index64, bool weighted,
   }
 }
 
-// Groups of at least this many (table, sample, column tile) items use the
-// row-stream kernel by default.
+// Groups of at least this many (table, sample, column tile) items use the row-stream
+// kernel whatever their rows per bag; smaller ones as pick_kernel says.
 constexpr int64_t kStreamMinBags = int64_t(1) << 20;
+constexpr int64_t kStreamBagsPerRow = 49152;
+constexpr int64_t kAnyRowsPerBag = 24;
 
 // Rows a wave of the row-stream kernel should walk: measured on 200 INT4 tables x
 // 32768 bags of ~40 rows, 32 bags per wave (1280 rows) ran 3.14 ms, 24 or 40 bags
@@ -282,18 +284,70 @@ KernelFn pooled_kernel_for(const TbePlanGroup& g, bool index64, bool weighted, b
 // every type and width (tbe_kern_any.hip) instead of a launch per group: 15 launches of
 // 5 us kernels cost ~95 us whatever the batch.  64 mixed tables (weighted mean, 32 rows
 // a bag): 2 k bags 93 -> 7 us, 32 k bags 95 -> 33, 131 k bags 182 -> 132, 262 k bags
-// 286 -> 266; past it the specialised kernels' pipeline over bags wins (524 k bags 461
-// against 516 us).
-constexpr int64_t kAnyMaxBags = int64_t(1) << 18;
+// 286 -> 266, 524 k bags 461 -> 516.  The line is at half of the crossing because short
+// bags cross earlier (its waves take ~0.5 ns a bag however short, the others ~0.2).
+constexpr int64_t kAnyMaxBags = int64_t(1) << 17;
+
+// the flags that choose a kernel per group keep doing so
+constexpr int32_t kKernelFlags = TBE_FLAG_NO_STREAM | TBE_FLAG_FORCE_STREAM | TBE_FLAG_NARROW_WORDS;
 
 bool use_any_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan) {
-  // the flags that choose a kernel per group keep doing so
-  if (a->flags & (TBE_FLAG_NO_STREAM | TBE_FLAG_FORCE_STREAM | TBE_FLAG_NARROW_WORDS)) return false;
+  if (a->flags & kKernelFlags) return false;
   if (plan.num_groups < 2 || a->num_indices > 0x7FFFFFFF || static_cast<int64_t>(a->T) * a->B > kAnyMaxBags)
     return false;
   for (int gi = 0; gi < plan.num_groups; ++gi)  // 32-bit row offsets only
     if (!plan.groups[gi].offset32) return false;
   return true;
+}
+
+// The kernel of one group: per-bag, row-stream or the any-type kernel, by the group's
+// bags, rows per bag and row width.  The lines lie where 16 tables of that shape crossed
+// (Zipf 1.05; us as per-bag / row-stream / any):
+//  * Row streams share a wave's set-up among its bags, so they win where bags are short
+//    and many.  Rows up to 32 words: from ~49 k bags per row of a bag (INT8 D 64, 524 k
+//    bags: 2 rows 93 / 42, 5 rows 106 / 66, 12 rows 122 / 109, 30 rows 207 / 214; 131 k
+//    bags: 2 rows 28 / 24, 5 rows 29 / 29), and always from 2^20 bags x column tiles.
+//  * Rows of 33-128 words, plain float: FP32 D 128, 8 k bags: 12 rows 12 / 10 / 11, 30
+//    rows 17 / 17 / 16; 131 k bags: 5 rows 82 / 39 / 75, 30 rows 220 / 189 / 208, 60 rows
+//    392 / 350 / 347.  INT8 and FP8 rows, which cost more to decode: INT8 D 512, 8 k bags:
+//    5 rows 12 / 11 / 11; 32 k bags: 5 rows 29 / 24 / 28, 12 rows 41 / 37 / 39, 30 rows
+//    84 / 83 / 78; 131 k bags: 12 rows 163 / 136 / 175, 30 rows 301 / 265 / 284.
+//  * Rows past 128 words: the any kernel reads 256 words of a row at a time (FP8 D 1024,
+//    32 k bags: 5 rows 53 / 42 / 32, 30 rows 154 / 129 / 100; FP32 D 512: 30 rows 234 /
+//    200 / 153), all but the shortest plain-float bags (131 k bags, 2 rows 267 / 85 / 153).
+//  * Else rows of 33 words or more take the any kernel from about 24 rows a bag, where its
+//    waves ending with their bag beats the persistent pipeline (INT8 D 256, 32 k bags: 5
+//    rows 17 / 16 / 19, 30 rows 42 / 44 / 38, 60 rows 78 / 84 / 67).  INT2 rows keep one
+//    word per lane in it (16 sums a word) and gain nothing.  Not beside other groups of
+//    a large call, whose persistent kernels its waves crowd out (64 mixed tables, 1 M bags
+//    of 32 rows: 789 -> 832 us; of 5 rows, with the row streams above: 486 -> 399).
+enum class Pool { kBag, kStream, kAny };
+
+Pool pick_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const TbePlanGroup& g, int64_t rows_per_bag) {
+  if (!g.offset32 || a->num_indices > 0x7FFFFFFF) return Pool::kBag;
+  const bool stream = g.stream && !(a->flags & TBE_FLAG_NO_STREAM);
+  const bool many = static_cast<int64_t>(g.count) * a->B * g.col_tiles >= kStreamMinBags;
+  if (a->flags & kKernelFlags)
+    return stream && (many || (a->flags & TBE_FLAG_FORCE_STREAM)) ? Pool::kStream : Pool::kBag;
+  const bool alone = plan.num_groups == 1;
+  const int64_t bags = static_cast<int64_t>(a->T) * a->B;  // the groups of a call share the GPU
+  const bool plain = g.weight_ty == TBE_TY_FP32 || g.weight_ty == TBE_TY_FP16 || g.weight_ty == TBE_TY_BF16;
+  const bool bytes = g.weight_ty == TBE_TY_INT8 || g.weight_ty == TBE_TY_FP8;
+  if (g.log2_lanes == 6 && (plain || bytes)) {
+    if (g.col_tiles > 2)
+      return stream && plain && rows_per_bag <= 8 && bags >= (1 << 15) ? Pool::kStream : Pool::kAny;
+    const int64_t few = plain ? (1 << 13) : (1 << 15);
+    const int64_t all = plain && g.col_tiles == 1 ? (1 << 15) : (1 << 17);
+    if (stream && (many || (bags >= few && rows_per_bag <= (plain ? 16 : 12)) ||
+                   (alone && bags >= all && rows_per_bag <= (plain ? 40 : 24))))
+      return Pool::kStream;
+    return alone && (g.col_tiles > 1 || rows_per_bag >= kAnyRowsPerBag) ? Pool::kAny : Pool::kBag;
+  }
+  if (stream && (many || bags >= kStreamBagsPerRow * std::max<int64_t>(1, rows_per_bag))) return Pool::kStream;
+  if (alone && g.weight_ty == TBE_TY_INT4 && g.log2_lanes == 6 &&
+      rows_per_bag >= kAnyRowsPerBag * (a->indice_weights ? 2 : 1))
+    return Pool::kAny;
+  return Pool::kBag;
 }
 
 // Four waves per bag instead of one when bags are long and too few to fill the GPU
@@ -394,6 +448,16 @@ hipError_t launch(KernelFn fn, KParams& p, int64_t want_blocks, bool persistent,
   void* args[] = {&p};
   return hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3(static_cast<uint32_t>(blocks)), dim3(kBlock),
                          args, 0, s);
+}
+
+// The one kernel over `items` bags x column tiles: the group p describes, or every
+// table (p.order null).
+hipError_t launch_any(KParams& p, int64_t items, int tiles, bool weighted, bool split, hipStream_t s) {
+  p.col_tiles = tiles;
+  p.div_tiles = make_fastdiv(static_cast<uint32_t>(tiles));
+  p.num_items = static_cast<int32_t>(items);
+  return launch(any_kernel(p.index64 != 0, weighted, split), p,
+                split ? items : (items + kWavesPerBlock - 1) / kWavesPerBlock, false, s);
 }
 
 }  // namespace tbe
@@ -617,17 +681,14 @@ int tbe_nbit_forward(const TbeNbitArgs* a, void* hip_stream) {
   const bool weighted = a->indice_weights != nullptr;
   // the per-group kernels keep index positions in 32 bits
   const bool wide = a->num_indices > 0x7FFFFFFF;
+  const int64_t rows_per_bag = a->num_indices / nbags;
   if (use_any_kernel(a, plan)) {
     int tiles = 1;
     for (int gi = 0; gi < plan.num_groups; ++gi)
       tiles = std::max(tiles, any_col_tiles(plan.groups[gi].weight_ty, plan.groups[gi].col_tiles));
-    const int64_t items = nbags * tiles;
-    const bool split = any_split(items, a->num_indices / nbags);
-    p.col_tiles = tiles;
-    p.div_tiles = make_fastdiv(static_cast<uint32_t>(tiles));
-    p.num_items = static_cast<int32_t>(items);
-    const hipError_t err = launch(any_kernel(p.index64 != 0, weighted, split), p,
-                                  split ? items : (items + kWavesPerBlock - 1) / kWavesPerBlock, false, s);
+    p.order = nullptr;
+    const hipError_t err =
+        launch_any(p, nbags * tiles, tiles, weighted, any_split(nbags * tiles, rows_per_bag), s);
     if (err != hipSuccess) return fail(TBE_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
     return TBE_OK;
   }
@@ -676,17 +737,18 @@ int tbe_nbit_forward(const TbeNbitArgs* a, void* hip_stream) {
     p.group_count = g.count;
     p.col_tiles = g.col_tiles;
     p.div_tiles = make_fastdiv(static_cast<uint32_t>(g.col_tiles));
-    // row streams pay off on large groups (measured: 200 tables x 32768 bags, 25 %
-    // faster); the per-bag kernel is as fast or faster below about a million bags
     const int64_t group_bags = static_cast<int64_t>(g.count) * a->B * g.col_tiles;
-    const bool use_stream = g.stream && !(a->flags & TBE_FLAG_NO_STREAM) &&
-                            ((a->flags & TBE_FLAG_FORCE_STREAM) || group_bags >= kStreamMinBags);
-    if (!wide && use_stream) {
+    const Pool pool = pick_kernel(a, plan, g, rows_per_bag);
+    if (pool == Pool::kAny) {
+      // a wave per item adds a wide row's bag in index order, as the other kernels do
+      const int tiles = any_col_tiles(g.weight_ty, g.col_tiles);
+      err = launch_any(p, static_cast<int64_t>(g.count) * a->B * tiles, tiles, weighted, false, gstream);
+    } else if (pool == Pool::kStream) {
       // one wave per (table, range of bags, column tile), no persistence
       const KernelFn fn = stream_kernel_group(g, p.index64 != 0, weighted, p.fp8);
-      const double rows_per_bag = static_cast<double>(a->num_indices) / static_cast<double>(std::max<int64_t>(1, a->T * a->B));
+      const double mean_rows = static_cast<double>(a->num_indices) / static_cast<double>(nbags);
       p.bags_per_wave = stream_bags_per_wave(group_bags,
-                                             static_cast<int64_t>(resident_blocks(fn)) * kWavesPerBlock, rows_per_bag);
+                                             static_cast<int64_t>(resident_blocks(fn)) * kWavesPerBlock, mean_rows);
       p.ranges = static_cast<int32_t>((a->B + p.bags_per_wave - 1) / p.bags_per_wave);
       p.div_ranges = make_fastdiv(static_cast<uint32_t>(p.ranges));
       const int64_t items = static_cast<int64_t>(g.count) * p.ranges * g.col_tiles;
