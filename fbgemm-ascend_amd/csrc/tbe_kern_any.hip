@@ -20,8 +20,11 @@
 //    value.  Rows of more than 64 payload words are read 2 or 4 words per lane
 //    (at most 16 accumulators a lane), so a row of up to 1 KiB is one item instead
 //    of one per 256 bytes (12 float tables, 24.6 k bags: 113 -> 37 us).
-//  * 8 row loads per lane and step, 4 of four words: 5-6 waves per SIMD.  8 of four
+//  * 8 row loads per lane and step, 4 of several words: 5-6 waves per SIMD.  8 of four
 //    words leave 4 waves and cost more than they hide (the same call 37 -> 44 us).
+//  * INT4 rows of 17-32 words take 16 lanes of two words, as in the per-bag kernel: four
+//    rows a load instead of two, and sums over four slots (64 mixed tables, 128 k bags:
+//    132 -> 113 us, error against 64-bit sums 3.4e-7 -> 3.2e-7).
 #include "tbe_kernels.h"
 
 namespace tbe {
@@ -60,10 +63,12 @@ __device__ __forceinline__ void any_bag(const KParams& p, const TbeTableDesc& td
   constexpr int EW = Traits<WT>::kEpd;
   constexpr int E = EW * VW;
   constexpr bool HDR = Traits<WT>::kHdr;
-  constexpr int U = VW == 4 ? 4 : 8;  // row loads per lane and step
+  constexpr int U = VW == 4 || (WT == TBE_TY_INT4 && VW == 2) ? 4 : 8;  // row loads per lane and step
   const int lane = threadIdx.x & (kWave - 1);
-  // lanes per row: at least 8, so that a step's R * U rows fit the 64 lanes that hold its indices
-  const int lg = VW == 1 ? max(static_cast<int>(td.log2_lanes), 3) : 6;
+  // lanes per row: at least 8, so that a step's R * U rows fit the 64 lanes that hold its
+  // indices; 16 for the INT4 rows of 17-32 words that are read two words per lane
+  constexpr bool kHalf = WT == TBE_TY_INT4 && VW == 2;
+  const int lg = VW == 1 ? max(static_cast<int>(td.log2_lanes), 3) : (kHalf && td.log2_lanes == 5 ? 4 : 6);
   const int R = kWave >> lg;
   const int S = R * U;
   const int slot = lane >> lg;
@@ -139,7 +144,7 @@ __device__ __forceinline__ void any_bag(const KParams& p, const TbeTableDesc& td
     }
   }
 
-  if constexpr (VW == 1) reduce_slots<E, HDR>(acc, bacc, lg);
+  if constexpr (VW == 1 || kHalf) reduce_slots<E, HDR>(acc, bacc, lg);
   if constexpr (WPB > 1) {
     const int wv = uniform(threadIdx.x >> 6);
     if (wv > 0) {
@@ -179,7 +184,8 @@ __device__ __forceinline__ void any_table(const KParams& p, const TbeTableDesc& 
                                           int ct, int64_t b, AnyShared<WPB>& sh) {
   constexpr int MV = any_max_vw<WT>();
   const int words = td.data_dwords;
-  if (MV == 1 || words <= kWave) {
+  const bool half = WT == TBE_TY_INT4 && td.log2_lanes == 5;
+  if (MV == 1 || (words <= kWave && !half)) {
     if (ct * kWave < words) any_bag<WT, 1, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh);
   } else if (MV == 2 || words <= 2 * kWave) {
     if (ct * 2 * kWave < words) any_bag<WT, MV < 2 ? 1 : 2, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh);

@@ -283,8 +283,8 @@ KernelFn pooled_kernel_for(const TbePlanGroup& g, bool index64, bool weighted, b
 // Calls of several table groups with at most this many bags take the one kernel for
 // every type and width (tbe_kern_any.hip) instead of a launch per group: 15 launches of
 // 5 us kernels cost ~95 us whatever the batch.  64 mixed tables (weighted mean, 32 rows
-// a bag): 2 k bags 93 -> 7 us, 32 k bags 95 -> 33, 131 k bags 182 -> 132, 262 k bags
-// 286 -> 266, 524 k bags 461 -> 516.  The line is at half of the crossing because short
+// a bag): 2 k bags 93 -> 7 us, 32 k bags 95 -> 32, 128 k bags 156 -> 113, 524 k bags
+// 461 -> 516.  The line is at half of the crossing because short
 // bags cross earlier (its waves take ~0.5 ns a bag however short, the others ~0.2).
 constexpr int64_t kAnyMaxBags = int64_t(1) << 17;
 

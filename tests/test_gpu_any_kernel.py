@@ -9,9 +9,9 @@ from test_gpu_parity import BF16, FP8, FP16, FP32, INT2, INT4, INT8, _check_modu
 pytestmark = pytest.mark.gpu
 
 PER_WORD = {FP32: 1, FP16: 2, BF16: 2, FP8: 4, INT8: 4, INT4: 8, INT2: 16}
-# payload words: 1-4 lanes, a full tile and one past it, two and four words per lane with
-# a cut last lane, more than one tile of four
-WORDS = (1, 3, 5, 63, 64, 65, 127, 129, 131, 257)
+# payload words: 1-4 lanes, INT4's half rows, a full tile and one past it, two and four
+# words per lane with a cut last lane, more than one tile of four
+WORDS = (1, 3, 5, 16, 17, 32, 33, 63, 64, 65, 127, 129, 131, 257)
 
 
 @pytest.mark.parametrize("lengths", ["short", "long"])
