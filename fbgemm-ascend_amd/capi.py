@@ -16,7 +16,7 @@ from . import HIP_LIB
 ABI_VERSION = 3
 EXPORTS = ("tbe_nbit_plan", "tbe_nbit_forward", "tbe_last_error", "tbe_nbit_abi_version",
            "tbe_permute_pooled_embs", "tbe_block_bucketize_workspace_bytes",
-           "tbe_block_bucketize_sparse_features", "tbe_block_bucketize_sparse_features_noalloc")
+           "tbe_block_bucketize_store_lists", "tbe_block_bucketize_sparse_features", "tbe_block_bucketize_sparse_features_noalloc")
 # TBE_BLOCK_BUCKETIZE_NOALLOC_SCRATCH_BYTES of include/tbe_sparse_ops.h
 NOALLOC_SCRATCH_BYTES = 32 << 20
 

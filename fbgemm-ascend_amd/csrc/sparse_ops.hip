@@ -363,6 +363,20 @@ __device__ __forceinline__ uint64_t lanes_with_bucket(const BucketBits<NB>& bb, 
   return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
+// Entries of the position lists handed over in one launch's arguments.
+constexpr int kListArgs = 120;
+struct ListArgs {
+  const void* ptr[kListArgs];
+  int64_t len[kListArgs];
+};
+
+__global__ void bb_store_lists(ListArgs a, int32_t n, int64_t* __restrict__ ptr, int64_t* __restrict__ len) {
+  const int i = threadIdx.x;
+  if (i >= n) return;
+  ptr[i] = reinterpret_cast<int64_t>(a.ptr[i]);
+  len[i] = a.len[i];
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBBBlock) void bb_fill_zero(T* __restrict__ a, int64_t n, uint32_t* __restrict__ b,
                                                         int64_t nb) {
@@ -673,35 +687,36 @@ __device__ __forceinline__ void scatter_row_atomic(const BBParams<IT, OT>& p, co
 // flags (`slow`, one byte per row) the rows it leaves: those not marked fast and
 // those holding an index at or above gsize; 2 takes the flagged rows with the
 // general map.  Two kernels, so the general map's registers do not limit the fast
-// pass.  my_size > 64: PASS 0, every row.
+// pass.  PASS 0, every row: my_size > 64, and calls with bucket boundaries.
 template <typename IT, typename OT, int NB, int PASS>
 __global__ __launch_bounds__(kBBBlock) void bb_scatter(BBParams<IT, OT> p) {
   __shared__ ScatterStage<IT> lds_stage[NB > 0 ? kBBBlock / kWaveBB : 1];
   ScatterStage<IT>& st = lds_stage[NB > 0 ? (threadIdx.x >> 6) : 0];
   if constexpr (NB > 0) st.cnt[lane_id()] = 0;
-  int64_t r0, r1, rs;
   if constexpr (PASS == 2) {
-    // few rows if any: each wave checks 64 consecutive rows' flags at a time
+    // few rows if any: each wave checks up to 64 rows' flags at a time.  Its rows are a
+    // grid's waves apart, so that flagged neighbours (a whole feature's rows) spread over
+    // the waves: one wave taking 64 consecutive rows left 983 k indices of 12 k flagged
+    // rows to 192 waves, 203 us.
     const int64_t waves = static_cast<int64_t>(gridDim.x) * (kBBBlock / kWaveBB);
-    r0 = (static_cast<int64_t>(blockIdx.x) * (kBBBlock / kWaveBB) + (threadIdx.x >> 6)) * kWaveBB;
-    r1 = p.L;
-    rs = 1;
-    for (int64_t g0 = r0; g0 < r1; g0 += waves * kWaveBB) {
-      const int64_t rl = g0 + lane_id();
-      uint64_t take = __builtin_amdgcn_ballot_w64(rl < r1 && p.slow[rl] != 0);
+    const int64_t w0 = static_cast<int64_t>(blockIdx.x) * (kBBBlock / kWaveBB) + (threadIdx.x >> 6);
+    for (int64_t g0 = w0; g0 < p.L; g0 += waves * kWaveBB) {
+      const int64_t rl = g0 + lane_id() * waves;
+      uint64_t take = __builtin_amdgcn_ballot_w64(rl < p.L && p.slow[rl] != 0);
       if (take == 0) continue;  // wave-uniform
-      const RowCtx<IT> mine = row_ctx_lane(p, rl < r1 ? rl : -1);
+      const RowCtx<IT> mine = row_ctx_lane(p, rl < p.L ? rl : -1);
       while (take) {
         const int j = __builtin_ctzll(take);
         take &= take - 1;
         const RowCtx<IT> c = row_ctx_of(mine, j);
         if (!c.ok) continue;
-        if (c.fast) scatter_row_staged<true, NB>(p, c, g0 + j, st);
-        else scatter_row_staged<false, NB>(p, c, g0 + j, st);
+        if (c.fast) scatter_row_staged<true, NB>(p, c, g0 + j * waves, st);
+        else scatter_row_staged<false, NB>(p, c, g0 + j * waves, st);
       }
     }
     return;
   }
+  int64_t r0, r1, rs;
   wave_rows(p.L, r0, r1, rs, true);
   for (int64_t g0 = r0; g0 < r1; g0 += kWaveBB * rs) {
     const int64_t rl = g0 + lane_id() * rs;
@@ -1005,10 +1020,15 @@ int run(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_of
   }
   if (p.N > 0) {
     const dim3 g(static_cast<uint32_t>(row_blocks));
-    // the general pass: one wave per 64 rows, at most one block per CU
-    const dim3 g2(static_cast<uint32_t>(std::min<int64_t>(std::max<int64_t>(1, (p.L + 255) / 256), cus)));
+    // the general pass: the first pass's waves, at most four blocks per CU
+    const dim3 g2(static_cast<uint32_t>(std::min<int64_t>(row_blocks, 4LL * cus)));
     if (!reg) {
       hipLaunchKernelGGL((bb_scatter<IT, OT, 0, 0>), g, dim3(kBBBlock), 0, s, p);
+    } else if (p.pos) {
+      // bucket boundaries given: every row takes the general map, in one pass (96 features
+      // x 128 rows, 983 k int32 indices: 8 + 203 us in two passes)
+      if (nbits <= 4) hipLaunchKernelGGL((bb_scatter<IT, OT, 4, 0>), g, dim3(kBBBlock), 0, s, p);
+      else hipLaunchKernelGGL((bb_scatter<IT, OT, 6, 0>), g, dim3(kBBBlock), 0, s, p);
     } else if (nbits <= 4) {
       hipLaunchKernelGGL((bb_scatter<IT, OT, 4, 1>), g, dim3(kBBBlock), 0, s, p);
       hipLaunchKernelGGL((bb_scatter<IT, OT, 4, 2>), g2, dim3(kBBBlock), 0, s, p);
@@ -1071,6 +1091,26 @@ int dispatch(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t su
 
 }  // namespace
 }  // namespace tbe
+
+extern "C" int tbe_block_bucketize_store_lists(const void* const* lists, const int64_t* lens, int32_t num_features,
+                                               void* out, void* hip_stream) {
+  clear_error();
+  if (num_features <= 0 || !lists || !lens || !out) return fail(TBE_ERR_INVALID_ARG, "bad position lists");
+  int64_t* ptr = static_cast<int64_t*>(out);
+  for (int32_t f = 0; f < num_features; f += kListArgs) {
+    ListArgs a;
+    const int32_t n = std::min(kListArgs, num_features - f);
+    for (int32_t i = 0; i < n; ++i) {
+      a.ptr[i] = lists[f + i];
+      a.len[i] = lens[f + i];
+    }
+    hipLaunchKernelGGL(bb_store_lists, dim3(1), dim3(128), 0, static_cast<hipStream_t>(hip_stream), a, n, ptr + f,
+                       ptr + num_features + f);
+  }
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return fail(TBE_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+  return TBE_OK;
+}
 
 extern "C" int tbe_block_bucketize_sparse_features(const TbeBlockBucketizeArgs* a, void* hip_stream) {
   clear_error();

@@ -358,6 +358,7 @@ block_bucketize_sparse_features_hip(const Tensor& lengths, const Tensor& indices
     TORCH_CHECK(x->is_cuda() && x->get_device() == dev, name, " must be on the same HIP device as lengths");
 
   at::OptionalDeviceGuard guard(at::device_of(lengths));
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(dev).stream();
   const Tensor len_c = lengths.contiguous();
   const Tensor idx_c = indices.contiguous();
   const Tensor bs_c = block_sizes.contiguous();
@@ -372,7 +373,7 @@ block_bucketize_sparse_features_hip(const Tensor& lengths, const Tensor& indices
   Tensor bso;
   if (batch_size_per_feature.has_value())  // BA:172: complete cumsum
     bso = at::cat({at::zeros({1}, lopt), at::cumsum(batch_size_per_feature->contiguous(), 0, len_c.scalar_type())}).contiguous();
-  Tensor w_c, new_w, new_pos, unb, tnb_c, pos_ptrs, pos_lens;
+  Tensor w_c, new_w, new_pos, unb, tnb_c, pos_lists;
   std::vector<Tensor> pos_keep;
   if (weights.has_value()) {
     w_c = weights->contiguous();
@@ -384,18 +385,20 @@ block_bucketize_sparse_features_hip(const Tensor& lengths, const Tensor& indices
   if (block_bucketize_pos.has_value()) {
     TORCH_CHECK(static_cast<int64_t>(block_bucketize_pos->size()) == F,
                 "block_bucketize_pos must hold one tensor per feature");
-    std::vector<int64_t> ptrs(F), lens(F);
+    std::vector<const void*> ptrs(F);
+    std::vector<int64_t> lens(F);
     for (int64_t f = 0; f < F; ++f) {
       const Tensor& t = (*block_bucketize_pos)[f];
       TORCH_CHECK(t.scalar_type() == idx_c.scalar_type(), "block_bucketize_pos dtype must match indices.");
       TORCH_CHECK(t.is_cuda() && t.get_device() == dev, "block_bucketize_pos must be on the same HIP device");
       pos_keep.push_back(t.contiguous());
-      ptrs[f] = reinterpret_cast<int64_t>(pos_keep.back().data_ptr());
+      ptrs[f] = pos_keep.back().data_ptr();
       lens[f] = t.dim() == 1 ? t.numel() : 0;
     }
-    auto cpu64 = at::TensorOptions().dtype(at::kLong);
-    pos_ptrs = at::tensor(ptrs, cpu64).to(len_c.device());
-    pos_lens = at::tensor(lens, cpu64).to(len_c.device());
+    pos_lists = at::empty({2 * F}, lopt.dtype(at::kLong));
+    const int rc = tbe_block_bucketize_store_lists(ptrs.data(), lens.data(), static_cast<int32_t>(F),
+                                                   pos_lists.data_ptr(), stream);
+    TORCH_CHECK(rc == TBE_OK, "block_bucketize_sparse_features: ", tbe_last_error());
   }
   const int64_t ws_bytes = tbe_block_bucketize_workspace_bytes(my_size, L, static_cast<int32_t>(len_c.element_size()));
   TORCH_CHECK(ws_bytes > 0, "block_bucketize_sparse_features: bad sizes");
@@ -416,8 +419,8 @@ block_bucketize_sparse_features_hip(const Tensor& lengths, const Tensor& indices
   a.weights = w_c.defined() ? w_c.data_ptr<float>() : nullptr;
   a.batch_size_offsets = bso.defined() ? bso.data_ptr() : nullptr;
   a.total_num_blocks = tnb_c.defined() ? tnb_c.data_ptr() : nullptr;
-  a.bucketize_pos = pos_ptrs.defined() ? reinterpret_cast<const void* const*>(pos_ptrs.data_ptr()) : nullptr;
-  a.bucketize_pos_len = pos_lens.defined() ? pos_lens.data_ptr<int64_t>() : nullptr;
+  a.bucketize_pos = pos_lists.defined() ? reinterpret_cast<const void* const*>(pos_lists.data_ptr()) : nullptr;
+  a.bucketize_pos_len = pos_lists.defined() ? pos_lists.data_ptr<int64_t>() + F : nullptr;
   a.new_lengths = new_lengths.data_ptr();
   a.new_offsets = new_offsets.data_ptr();
   a.new_indices = new_indices.data_ptr();
@@ -426,7 +429,6 @@ block_bucketize_sparse_features_hip(const Tensor& lengths, const Tensor& indices
   a.unbucketize_permute = unb.defined() ? unb.data_ptr() : nullptr;
   a.workspace = ws.data_ptr();
   a.workspace_bytes = ws_bytes;
-  const hipStream_t stream = c10::hip::getCurrentHIPStream(dev).stream();
   const int rc = tbe_block_bucketize_sparse_features(&a, stream);
   TORCH_CHECK(rc == TBE_OK, "block_bucketize_sparse_features: ", tbe_last_error());
   auto opt = [](const Tensor& t) { return t.defined() ? c10::optional<Tensor>(t) : c10::nullopt; };

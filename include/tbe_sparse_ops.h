@@ -83,6 +83,16 @@ typedef struct TbeBlockBucketizeArgs {
 
 int64_t tbe_block_bucketize_workspace_bytes(int64_t my_size, int64_t lengths_size, int32_t offset_size);
 
+/*
+ * The two device arrays of the position lists from host arrays: writes the
+ * num_features list pointers (bucketize_pos) and then the num_features lengths
+ * (bucketize_pos_len) to out, device [2 * num_features] of 8 bytes, on the stream.
+ * The values travel as kernel arguments: no host copy that would make the caller wait,
+ * and nothing that has to outlive the call.
+ */
+int tbe_block_bucketize_store_lists(const void* const* lists, const int64_t* lens, int32_t num_features, void* out,
+                                    void* hip_stream);
+
 int tbe_block_bucketize_sparse_features(const TbeBlockBucketizeArgs* args, void* hip_stream);
 
 /*
