@@ -126,9 +126,11 @@ struct RowCtx {
 };
 
 // BK:322-347 (row -> feature) and BK:388-421 (per-feature parameters) for row r
-// of this lane; r < 0 gives ok = false.
+// of this lane; r < 0 gives ok = false.  `own`: the complete cumsum from row `own_first`
+// on, where the caller holds it, instead of p.offsets.
 template <typename IT, typename OT>
-__device__ __forceinline__ RowCtx<IT> row_ctx_lane(const BBParams<IT, OT>& p, int64_t r) {
+__device__ __forceinline__ RowCtx<IT> row_ctx_lane(const BBParams<IT, OT>& p, int64_t r, const OT* own = nullptr,
+                                                   int64_t own_first = 0) {
   using UIT = std::make_unsigned_t<IT>;
   RowCtx<IT> c{};
   c.ok = false;
@@ -176,8 +178,14 @@ __device__ __forceinline__ RowCtx<IT> row_ctx_lane(const BBParams<IT, OT>& p, in
   c.fast = !c.pos && blk > 0 && c.lsize > 0 && (static_cast<uint64_t>(c.gsize) >> 32) == 0 &&
            (static_cast<uint64_t>(c.lsize) >> 32) == 0;
   c.dl = make_fastdiv(c.fast ? static_cast<uint32_t>(c.lsize) : 1u);
-  int64_t s = r == 0 ? 0 : static_cast<int64_t>(p.offsets[r - 1]);
-  int64_t e = static_cast<int64_t>(p.offsets[r]);
+  int64_t s, e;
+  if (own) {
+    s = static_cast<int64_t>(own[r - own_first]);
+    e = static_cast<int64_t>(own[r - own_first + 1]);
+  } else {
+    s = r == 0 ? 0 : static_cast<int64_t>(p.offsets[r - 1]);
+    e = static_cast<int64_t>(p.offsets[r]);
+  }
   s = std::min<int64_t>(std::max<int64_t>(s, 0), p.N);  // malformed offsets never read out of bounds
   e = std::min<int64_t>(std::max<int64_t>(e, s), p.N);
   c.s = s;
@@ -556,10 +564,11 @@ __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t x) {
 // ONLY_FAST (rows marked fast): gives up on the row, returning false, at the
 // first chunk holding an index at or above gsize, before writing anything of that
 // chunk; the general pass then rewrites the whole row (the same values at the same
-// positions).  Returns true when the row is done.
+// positions).  Returns true when the row is done.  `cur`: the row's first output offset
+// per bucket where the caller holds it, instead of p.new_offsets.
 template <bool FAST, int NB, typename IT, typename OT, bool ONLY_FAST = false>
 __device__ __forceinline__ bool scatter_row_staged(const BBParams<IT, OT>& p, const RowCtx<IT>& c, int64_t r,
-                                                   ScatterStage<IT>& st) {
+                                                   ScatterStage<IT>& st, const int64_t* cur = nullptr) {
   using UIT = std::make_unsigned_t<IT>;
   constexpr uint32_t kNone = 0xFFu;
   const UIT* __restrict__ idx = reinterpret_cast<const UIT*>(p.indices);
@@ -570,7 +579,8 @@ __device__ __forceinline__ bool scatter_row_staged(const BBParams<IT, OT>& p, co
     for (int k = 0; k < kChunk; ++k)  // clamped, not branched: the row is not empty
       uk[k] = idx[std::min<int64_t>(chunk + k * kWaveBB + lane, c.e - 1)];
     // the row's cursors, loaded with its first indices (one wait for both)
-    if (chunk == c.s && lane < p.my_size) st.cur[lane] = static_cast<int64_t>(p.new_offsets[lane * p.L + r]);
+    if (chunk == c.s && lane < p.my_size)
+      st.cur[lane] = cur ? cur[lane] : static_cast<int64_t>(p.new_offsets[lane * p.L + r]);
     if constexpr (ONLY_FAST) {
       bool high = false;
 #pragma unroll
@@ -863,6 +873,161 @@ __global__ __launch_bounds__(kBBBlock) void scan_tiles_based(const T* __restrict
   if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = T(0);
 }
 
+// ---------------------------------------------------------------- few rows: two launches
+//
+// Up to a few thousand rows the call above is six or seven launches of 2-7 us kernels,
+// bound by launching.  Here the two scans are folded into the two kernels that need them:
+// a work-group of the count sums the lengths before its rows itself, and a work-group of
+// the scatter sums the bucket totals that the count's work-groups left (my_size x groups
+// values, from L2) instead of scanning my_size x L counts.  48 features x 32 rows, 12 ranks
+// (37 k weighted int64 indices): 28.2 -> 15.9 us.
+
+constexpr int kFewRowsMax = 16;  // rows of one work-group
+
+template <typename IT, typename OT>
+__global__ __launch_bounds__(kBBBlock) void bb_count_few(BBParams<IT, OT> p, const OT* __restrict__ lengths,
+                                                        OT* __restrict__ formed, OT* __restrict__ sums, int per) {
+  __shared__ uint32_t lds_hist[kBBBlock / kWaveBB][kWaveBB];
+  __shared__ uint32_t group_sum[kWaveBB];
+  __shared__ OT own[kFewRowsMax + 1];
+  __shared__ OT lds_wave[kBBBlock / kWaveBB];
+  constexpr int kWaves = kBBBlock / kWaveBB;
+  const int lane = lane_id();
+  const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  uint32_t* hist = lds_hist[wv];
+  hist[lane] = 0;
+  if (wv == 0) group_sum[lane] = 0;
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * per;
+  const int n = static_cast<int>(std::min<int64_t>(per, p.L - b0));
+  if (lengths) {
+    OT part = 0;
+#pragma unroll 4
+    for (int64_t r = threadIdx.x; r < b0; r += kBBBlock) part += lengths[r];
+    OT base;
+    (void)block_exclusive_scan(part, lds_wave, base);
+    if (wv == 0) {
+      OT x = lane < n ? lengths[b0 + lane] : OT(0);
+#pragma unroll
+      for (int d = 1; d < kFewRowsMax; d <<= 1) {
+        const OT y = __shfl_up(x, d, kWaveBB);
+        if (lane >= d) x += y;
+      }
+      if (lane < n) {
+        own[lane + 1] = base + x;
+        formed[b0 + lane + 1] = base + x;
+      }
+      if (lane == 0) {
+        own[0] = base;
+        if (b0 == 0) formed[0] = OT(0);
+      }
+    }
+  }
+  __syncthreads();
+  // this wave's rows: b0 + wv, then every kWaves-th
+  const int mine_i = wv + lane * kWaves;
+  const RowCtx<IT> mine = row_ctx_lane(p, mine_i < n ? b0 + mine_i : -1, lengths ? own : nullptr, b0);
+  for (int j = 0; wv + j * kWaves < n; ++j) {
+    const int64_t r = b0 + wv + j * kWaves;
+    const RowCtx<IT> c = row_ctx_of(mine, j);
+    if (c.ok) {
+      if (c.fast) count_row<true, true>(p, c, r, hist, nullptr);
+      else count_row<false, true>(p, c, r, hist, nullptr);
+    }
+    const uint32_t cnt = hist[lane];  // the wave's LDS operations complete in order
+    hist[lane] = 0;
+    if (lane < p.my_size) p.new_lengths[lane * p.L + r] = static_cast<OT>(cnt);
+    atomicAdd(group_sum + lane, cnt);
+  }
+  __syncthreads();
+  if (wv == 0 && lane < p.my_size) sums[static_cast<int64_t>(lane) * gridDim.x + blockIdx.x] = static_cast<OT>(group_sum[lane]);
+}
+
+template <typename IT, typename OT, int NB>
+__global__ __launch_bounds__(kBBBlock) void bb_scatter_few(BBParams<IT, OT> p, const OT* __restrict__ sums, int per) {
+  __shared__ ScatterStage<IT> lds_stage[kBBBlock / kWaveBB];
+  __shared__ int64_t cur[kFewRowsMax][kWaveBB];
+  __shared__ OT total[kWaveBB], before[kWaveBB];  // per bucket: all rows, and the rows before this group's
+  constexpr int kWaves = kBBBlock / kWaveBB;
+  const int lane = lane_id();
+  const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  ScatterStage<IT>& st = lds_stage[wv];
+  st.cnt[lane] = 0;
+  const int my = static_cast<int>(p.my_size);
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * per;
+  const int n = static_cast<int>(std::min<int64_t>(per, p.L - b0));
+  // what the rows need besides the totals loads first, behind the sums below
+  const int mine_i = wv + lane * kWaves;
+  const RowCtx<IT> mine = row_ctx_lane(p, mine_i < n ? b0 + mine_i : -1);
+  OT cnt[kFewRowsMax];
+#pragma unroll
+  for (int i = 0; i < kFewRowsMax; ++i)
+    cnt[i] = wv == 0 && i < n && lane < my ? p.new_lengths[lane * p.L + b0 + i] : OT(0);
+  for (int b = wv; b < my; b += kWaves) {
+    OT all = 0, pre = 0;
+#pragma unroll 4
+    for (uint32_t i = lane; i < gridDim.x; i += kWaveBB) {
+      const OT v = sums[static_cast<int64_t>(b) * gridDim.x + i];
+      all += v;
+      pre += i < blockIdx.x ? v : OT(0);
+    }
+#pragma unroll
+    for (int d = kWaveBB / 2; d > 0; d >>= 1) {
+      all += __shfl_xor(all, d, kWaveBB);
+      pre += __shfl_xor(pre, d, kWaveBB);
+    }
+    if (lane == 0) {
+      total[b] = all;
+      before[b] = pre;
+    }
+  }
+  __syncthreads();
+  if (wv == 0) {  // lane = bucket: its first position, then its rows' offsets
+    const OT own = lane < my ? total[lane] : OT(0);
+    OT x = own;
+#pragma unroll
+    for (int d = 1; d < kWaveBB; d <<= 1) {
+      const OT y = __shfl_up(x, d, kWaveBB);
+      if (lane >= d) x += y;
+    }
+    if (lane < my) {
+      OT run = x - own + before[lane];
+      OT* out = const_cast<OT*>(p.new_offsets) + lane * p.L + b0;
+#pragma unroll
+      for (int i = 0; i < kFewRowsMax; ++i) {
+        if (i >= n) break;
+        cur[i][lane] = static_cast<int64_t>(run);
+        out[i] = run;
+        run += cnt[i];
+      }
+      if (b0 + n == p.L && lane == my - 1) out[n] = run;
+    }
+  }
+  __syncthreads();
+  for (int j = 0; wv + j * kWaves < n; ++j) {
+    const int i = wv + j * kWaves;
+    const RowCtx<IT> c = row_ctx_of(mine, j);
+    if (!c.ok) continue;
+    if (c.fast) scatter_row_staged<true, NB>(p, c, b0 + i, st, cur[i]);
+    else scatter_row_staged<false, NB>(p, c, b0 + i, st, cur[i]);
+  }
+}
+
+// Rows per work-group of the two launches, 0 where the general path is used.  The lines:
+// a work-group reads at most 16 k lengths and 16 k bucket totals, one row per wave while
+// the totals stay below 8 k (1536 rows, 12 ranks: 4 rows a group 15.9 us, 8 rows 17.4, 16
+// rows 21.8; 12288 rows, 8 ranks: 8 rows 47.3, 16 rows 44.6); past a million indices the general scatter's fast pass (more
+// waves per SIMD) is worth its launches (8192 rows, int64, 16 ranks: 2.6 M indices 43.8 us
+// against 45.6 in two launches; 12288 rows, 8 ranks, 983 k int32: 42.1 against 30.4), four
+// million with bucket boundaries, which the fast pass does not take.
+constexpr int64_t kFewIndices = int64_t(1) << 20;
+
+int few_rows_per_group(int64_t my, int64_t L, int64_t N, bool lists) {
+  if (my > kWaveBB || L < 1 || L > 16384 || N > (lists ? 4 : 1) * kFewIndices) return 0;
+  for (int per = 4; per <= kFewRowsMax; per *= 2)
+    if ((L + per - 1) / per * my <= (per < kFewRowsMax ? 8192 : 16384)) return per;
+  return 0;
+}
+
 int64_t scan_tiles_of(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
 
 // Bytes of the row offsets the library forms when the caller passes lengths only:
@@ -939,7 +1104,7 @@ int64_t noalloc_need(int64_t my, int64_t L, int32_t os, int64_t* sums_off) {
 }
 
 template <typename IT, typename OT>
-int run(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_off) {
+int run(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_off, void* few_sums, int64_t few_bytes) {
   BBParams<IT, OT> p{};
   p.indices = static_cast<const IT*>(a->indices);
   p.offsets = static_cast<const OT*>(a->offsets);
@@ -970,6 +1135,23 @@ int run(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_of
   p.keep = a->keep_orig_idx;
   int nbits = 0;  // ceil(log2(my_size))
   while (nbits < 6 && (int64_t(1) << nbits) < a->my_size) ++nbits;
+  const int per = few_rows_per_group(a->my_size, p.L, p.N, p.pos != nullptr);
+  if (per > 0) {
+    const int64_t groups = (p.L + per - 1) / per;
+    if (groups * a->my_size * static_cast<int64_t>(sizeof(OT)) <= few_bytes) {
+      OT* group_sums = static_cast<OT*>(few_sums);
+      const dim3 g(static_cast<uint32_t>(groups));
+      hipLaunchKernelGGL((bb_count_few<IT, OT>), g, dim3(kBBBlock), 0, s, p,
+                         a->offsets ? nullptr : static_cast<const OT*>(a->lengths), formed, group_sums, per);
+      if (nbits <= 4)
+        hipLaunchKernelGGL((bb_scatter_few<IT, OT, 4>), g, dim3(kBBBlock), 0, s, p, const_cast<const OT*>(group_sums), per);
+      else
+        hipLaunchKernelGGL((bb_scatter_few<IT, OT, 6>), g, dim3(kBBBlock), 0, s, p, const_cast<const OT*>(group_sums), per);
+      const hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return fail(TBE_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+      return TBE_OK;
+    }
+  }
   const int64_t nseg = a->my_size * a->lengths_size;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -1083,10 +1265,15 @@ int check_pointers(const TbeBlockBucketizeArgs* a) {
   return TBE_OK;
 }
 
-int dispatch(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_off) {
+// few_sums: scratch for the bucket totals of the two-launch path (few_bytes, may be too
+// small for it).
+int dispatch(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_off, void* few_sums,
+             int64_t few_bytes) {
   if (a->index_size == 4)
-    return a->offset_size == 4 ? run<int32_t, int32_t>(a, s, ws, sums_off) : run<int32_t, int64_t>(a, s, ws, sums_off);
-  return a->offset_size == 4 ? run<int64_t, int32_t>(a, s, ws, sums_off) : run<int64_t, int64_t>(a, s, ws, sums_off);
+    return a->offset_size == 4 ? run<int32_t, int32_t>(a, s, ws, sums_off, few_sums, few_bytes)
+                               : run<int32_t, int64_t>(a, s, ws, sums_off, few_sums, few_bytes);
+  return a->offset_size == 4 ? run<int64_t, int32_t>(a, s, ws, sums_off, few_sums, few_bytes)
+                             : run<int64_t, int64_t>(a, s, ws, sums_off, few_sums, few_bytes);
 }
 
 }  // namespace
@@ -1121,7 +1308,9 @@ extern "C" int tbe_block_bucketize_sparse_features(const TbeBlockBucketizeArgs* 
   if (!a->workspace || a->workspace_bytes < need)
     return fail(TBE_ERR_INVALID_ARG, "workspace of %lld bytes needed", static_cast<long long>(need));
   if (check_pointers(a) != TBE_OK) return TBE_ERR_INVALID_ARG;
-  return dispatch(a, static_cast<hipStream_t>(hip_stream), a->workspace, sums_off);
+  // the cursors' region, which the two-launch path does not otherwise use
+  const int64_t few_bytes = sums_off - offsets_bytes(a->lengths_size, a->offset_size);
+  return dispatch(a, static_cast<hipStream_t>(hip_stream), a->workspace, sums_off, a->workspace, few_bytes);
 }
 
 extern "C" int tbe_block_bucketize_sparse_features_noalloc(const TbeBlockBucketizeArgs* a, void* hip_stream) {
@@ -1150,7 +1339,9 @@ extern "C" int tbe_block_bucketize_sparse_features_noalloc(const TbeBlockBucketi
   const bool eager = cs == hipStreamCaptureStatusNone;
   if (eager && d->recorded && hipStreamWaitEvent(s, d->done, 0) != hipSuccess)
     return fail(TBE_ERR_LAUNCH, "hipStreamWaitEvent on the previous call failed");
-  const int rc2 = dispatch(a, s, d->scratch, sums_off);
+  const int64_t few_at = (need + 255) / 256 * 256;  // behind what the general path uses
+  const int rc2 = dispatch(a, s, d->scratch, sums_off, static_cast<uint8_t*>(d->scratch) + few_at,
+                           kNoAllocScratchBytes - few_at);
   if (eager && rc2 == TBE_OK) {
     if (hipEventRecord(d->done, s) != hipSuccess) return fail(TBE_ERR_LAUNCH, "hipEventRecord failed");
     d->recorded = true;

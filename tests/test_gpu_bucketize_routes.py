@@ -42,3 +42,38 @@ def test_rows_past_their_blocks(pkg, oracle, gpu, L):
     starts = np.cumsum(lengths) - lengths
     indices[starts[::2]] += 64 * 3
     _compare(oracle, gpu, lengths, indices, np.array([64], np.int32), 3)
+
+
+# the two-launch path: 4, 8 and 16 rows a work-group, cut last groups, the last sizes it
+# takes and the first it does not, the smallest calls
+@pytest.mark.parametrize("F,B,my,dtype", [
+    (1, 1, 1, np.int32), (1, 1, 33, np.int64), (1, 1, 64, np.int64), (3, 1, 2, np.int64), (7, 9, 64, np.int32),
+    (1, 2048, 16, np.int64), (1, 2049, 16, np.int64), (2, 2047, 32, np.int64), (1, 4097, 32, np.int64),
+    (1, 16384, 16, np.int32), (1, 16385, 16, np.int32), (5, 1639, 64, np.int64), (1, 300, 65, np.int64)])
+@pytest.mark.parametrize("lists", [False, True])
+def test_few_rows(pkg, oracle, gpu, F, B, my, dtype, lists):
+    rng = np.random.default_rng(F * B + my)
+    lengths = rng.integers(0, 12, F * B).astype(dtype)
+    lengths[:: max(1, F * B // 3)] = 700  # rows of more than one chunk
+    pos = [np.concatenate([[0], rng.integers(1, 50, my).cumsum()]).astype(dtype) for _ in range(F)] if lists else None
+    indices = rng.integers(0, 40 * my, int(lengths.sum())).astype(dtype)  # some past the blocks of 25
+    _compare(oracle, gpu, lengths, indices, np.full(F, 25, dtype), my, pos)
+
+
+@pytest.mark.parametrize("L", [1, 5, 4099])
+def test_few_rows_c_abi(pkg, oracle, gpu, L):
+    # offsets given or formed, scratch of the caller or the library's own; new_offsets is an output
+    rng = np.random.default_rng(L)
+    lengths = rng.integers(0, 9, L).astype(np.int64)
+    indices = rng.integers(0, 12, int(lengths.sum())).astype(np.int64)
+    want = oracle.block_bucketize_sparse_features(lengths, indices, False, True, np.array([4]), 3)
+    d = lambda a: torch.from_numpy(a).to(gpu)  # noqa: E731
+    for noalloc in (False, True):
+        for pass_offsets in (False, True):
+            got, offs = pkg.capi.block_bucketize_sparse_features(d(lengths), d(indices), False, True,
+                                                                 d(np.array([4])), 3, noalloc=noalloc,
+                                                                 pass_offsets=pass_offsets)
+            for g, e in zip(got, want):
+                if e is not None:
+                    assert np.array_equal(g.cpu().numpy(), e)
+            assert np.array_equal(offs.cpu().numpy(), np.concatenate([[0], want[0].cumsum()]))
