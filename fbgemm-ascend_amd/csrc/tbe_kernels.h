@@ -1416,8 +1416,21 @@ __device__ __forceinline__ void decode_word(uint32_t d, float (&v)[Traits<WT>::k
   }
 }
 
+// Rows whose segments are walked in rolled batches (nobag_segment) rather than with all
+// loads of a chunk unrolled.  us, 26 tables, 1.6 M indices unless said, unrolled -> batches:
+// INT8 D 64 / 128 80 -> 73 / 160 -> 131, FP8 D 64 / 128 70 -> 56 / 189 -> 105, FP16 D 64
+// 106 -> 55, FP32 D 16 36 -> 31, INT4 D 256 / 512 (0.8 / 0.4 M indices) 124 -> 84 /
+// 120 -> 86.  The others lose or draw: INT8 D 256 57 -> 62, BF16 D 128 154 -> 159, INT4
+// D 64 62 -> 64, INT2 D 256 170 -> 228.
+template <int WT, int LG>
+constexpr bool nobag_batches() {
+  if (WT == TBE_TY_INT2) return false;
+  if (WT == TBE_TY_INT4) return LG >= 5;
+  return LG == 4 || LG == 5;
+}
+
 template <int WT, int LG, typename IndexT, bool A64>
-__device__ __forceinline__ void nobag_segment(const KParams& p, const TbeTableDesc& td, int64_t a, int n) {
+__device__ __forceinline__ void nobag_segment_flat(const KParams& p, const TbeTableDesc& td, int64_t a, int n) {
   constexpr int E = Traits<WT>::kEpd;
   constexpr bool HDR = Traits<WT>::kHdr;
   constexpr int R = kWave >> LG;               // rows per load instruction
@@ -1476,6 +1489,140 @@ __device__ __forceinline__ void nobag_segment(const KParams& p, const TbeTableDe
   }
 }
 
+// Store E elements at byte `off` of a wave's output rows, non-temporally (see out_store).
+// `rs` covers exactly those rows, so rows past the segment are dropped by the range check.
+template <int E>
+__device__ __forceinline__ void store_rows(const KParams& p, __amdgpu_buffer_rsrc_t rs, uint32_t off,
+                                           const float (&r)[E]) {
+  constexpr int kNt = 2;  // cache policy of the buffer instructions: nt
+  const int o = static_cast<int>(off);
+  if (p.out_ty == TBE_TY_FP32) {
+    if constexpr (E % 4 == 0) {
+#pragma unroll
+      for (int i = 0; i < E; i += 4)
+        __builtin_amdgcn_raw_buffer_store_b128(tbe_u32x4{__float_as_uint(r[i]), __float_as_uint(r[i + 1]),
+                                                         __float_as_uint(r[i + 2]), __float_as_uint(r[i + 3])},
+                                               rs, o + 4 * i, 0, kNt);
+    } else if constexpr (E == 2) {
+      __builtin_amdgcn_raw_buffer_store_b64(tbe_u32x2{__float_as_uint(r[0]), __float_as_uint(r[1])}, rs, o, 0, kNt);
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(r[0]), rs, o, 0, kNt);
+    }
+    return;
+  }
+  uint16_t b[E];
+  if (p.out_ty == TBE_TY_FP16) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) b[i] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(r[i]));
+  } else {
+#pragma unroll
+    for (int i = 0; i < E; ++i) b[i] = static_cast<uint16_t>(f32_to_bf16_bits(r[i]));
+  }
+  if constexpr (E == 1) {
+    __builtin_amdgcn_raw_buffer_store_b16(b[0], rs, o, 0, kNt);
+  } else {
+    uint32_t w[E / 2];
+#pragma unroll
+    for (int i = 0; i < E / 2; ++i) w[i] = b[2 * i] | (uint32_t(b[2 * i + 1]) << 16);
+    if constexpr (E % 8 == 0) {
+#pragma unroll
+      for (int i = 0; i < E / 2; i += 4)
+        __builtin_amdgcn_raw_buffer_store_b128(tbe_u32x4{w[i], w[i + 1], w[i + 2], w[i + 3]}, rs, o + 4 * i, 0, kNt);
+    } else if constexpr (E == 4) {
+      __builtin_amdgcn_raw_buffer_store_b64(tbe_u32x2{w[0], w[1]}, rs, o, 0, kNt);
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b32(w[0], rs, o, 0, kNt);
+    }
+  }
+}
+
+// Rows of a segment go in batches of UB loads, the next batch loading while one is decoded
+// and stored, in a loop that is not unrolled further: with all 32 loads of a chunk unrolled
+// the INT8 kernel took 212 VGPRs, two waves per SIMD; now 64, eight.  26 INT8 tables D 128,
+// 1.6 M indices, fp16 out: 160 -> 132 us (Zipf 1.05), 167 -> 153 (uniform: 819 MB of lines
+// and output, 5.3 TB/s).  Batches of 4 loads 146 us, of 16 (256 VGPRs) 233.
+template <int WT, int LG, typename IndexT, bool A64>
+__device__ __forceinline__ void nobag_segment(const KParams& p, const TbeTableDesc& td, int64_t a, int n) {
+  constexpr int E = Traits<WT>::kEpd;
+  constexpr bool HDR = Traits<WT>::kHdr;
+  constexpr int R = kWave >> LG;               // rows per load instruction
+  constexpr int U = kWave / R;                 // load instructions per 64 rows
+  static_assert(U >= 16, "two trips of the loop at least: one is unrolled and takes 177 VGPRs");
+  constexpr int UB = U == 16 ? 4 : 8;          // issued together
+  const int lane = threadIdx.x & (kWave - 1);
+  const int slot = lane >> LG;
+  const uint32_t rows = static_cast<uint32_t>(td.num_rows);
+  const uint32_t stride = static_cast<uint32_t>(td.row_stride);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(p.weights + td.weights_offset), 0, static_cast<int>(rows * stride), kRsrcWord3);
+  const uint64_t raw = load_index_chunk<IndexT>(p, a, n);
+  const int64_t iv = sizeof(IndexT) == 8 ? static_cast<int64_t>(raw) : static_cast<int64_t>(static_cast<int32_t>(raw));
+  // A64: the row index (kNoRow64 for none); else the row's byte offset (kNoRow)
+  const bool has_row = lane < n && iv >= 0 && iv < static_cast<int64_t>(td.num_rows);
+  const uint32_t off = A64 ? (has_row ? static_cast<uint32_t>(iv) : kNoRow64)
+                           : (has_row ? static_cast<uint32_t>(iv) * stride : kNoRow);
+  const uint8_t* tbase = p.weights + td.weights_offset;
+  const bool vec = (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0 && p.out_stride % E == 0;
+  const uint32_t es = p.out_ty == TBE_TY_FP32 ? 4u : 2u;
+  const uint32_t out_row = static_cast<uint32_t>(uniform(static_cast<int>(static_cast<uint32_t>(p.out_stride) * es)));
+  const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
+      static_cast<uint8_t*>(p.out) + a * p.out_stride * es, 0, static_cast<int>(static_cast<uint32_t>(n) * out_row),
+      kRsrcWord3);
+  for (int ct = 0; ct < td.col_tiles; ++ct) {
+    const int dw = ct * kWave + (lane & ((1 << LG) - 1));
+    const bool col_ok = dw < td.data_dwords;
+    const uint32_t col = static_cast<uint32_t>(td.data_offset + (col_ok ? 4 * dw : 0));
+    const uint32_t ocol = static_cast<uint32_t>(slot) * out_row + static_cast<uint32_t>(dw) * E * es;
+    auto issue = [&](int u0, uint32_t from, uint32_t (&d)[UB], uint32_t (&h)[UB]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UB; ++u) {
+        const uint32_t o = static_cast<uint32_t>(
+            __builtin_amdgcn_ds_bpermute(((u0 + u) * R + slot) * 4, static_cast<int>(from)));
+        if constexpr (A64) {  // a lane without a row reads the zero row
+          const uint8_t* rp = o != kNoRow64 ? tbase + static_cast<uint64_t>(o) * stride
+                                            : reinterpret_cast<const uint8_t*>(g_zero_row);
+          d[u] = load_word(rp + col);
+          h[u] = HDR ? load_word(rp) : 0u;
+        } else {
+          d[u] = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(o + col), 0, 0));
+          h[u] = HDR ? static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(o), 0, 0)) : 0u;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto store = [&](int u0, const uint32_t (&d)[UB], const uint32_t (&h)[UB]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UB; ++u) {
+        if ((u0 + u) * R >= n) break;  // wave-uniform
+        float v[E], r[E];
+        decode_word<WT>(d[u], v, p.fp8);
+        // a rejected index reads a zero word and header: scale 0, bias 0 -> zeros
+        const float sc = HDR ? h16lo(h[u]) : 1.f, bi = HDR ? h16hi(h[u]) : 0.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) r[e] = HDR ? fmaf(sc, v[e], bi) : v[e];
+        if (vec && col_ok) {
+          store_rows<E>(p, ors, ocol + static_cast<uint32_t>((u0 + u) * R) * out_row, r);
+        } else if (col_ok) {
+          const int row = (u0 + u) * R + slot;
+          if (row < n) store_slice<E>(p, (a + row) * p.out_stride + static_cast<int64_t>(dw) * E, r, false);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t da[UB], ha[UB], db[UB], hb[UB];
+    issue(0, off, da, ha);
+#pragma unroll 1
+    for (int u0 = 0; u0 < U; u0 += 2 * UB) {
+      if (u0 * R >= n) break;  // wave-uniform
+      issue(u0 + UB, off, db, hb);
+      store(u0, da, ha);
+      // past the last batch: no rows, so that every path issues the same loads
+      issue(u0 + 2 * UB, u0 + 2 * UB < U ? off : (A64 ? kNoRow64 : kNoRow), da, ha);
+      store(u0 + UB, db, hb);
+    }
+  }
+}
+
 // Output rows of positions that no table's segment covers (before offsets[0], or
 // from offsets[T*B] on, e.g. when len(offsets)-1 is not a multiple of T) are
 // zero, as the reference's zero-initialised output leaves them (A:135).  One
@@ -1518,7 +1665,8 @@ __global__ __launch_bounds__(kBlock) void nobag_fast_kernel(KParams p) {
     const TbeTableDesc td = load_desc(p.tables + t);
     if (td.weight_ty != WT || td.log2_lanes != LG || ((td.flags & TBE_TABLE_OFFSET32) != 0) == A64) continue;
     if (A64 && td.num_rows >= static_cast<int64_t>(kNoRow64)) continue;  // the generic kernel's
-    nobag_segment<WT, LG, IndexT, A64>(p, td, a, static_cast<int>(e - a));
+    if constexpr (nobag_batches<WT, LG>()) nobag_segment<WT, LG, IndexT, A64>(p, td, a, static_cast<int>(e - a));
+    else nobag_segment_flat<WT, LG, IndexT, A64>(p, td, a, static_cast<int>(e - a));
   }
 }
 

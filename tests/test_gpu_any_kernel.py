@@ -42,3 +42,20 @@ def test_any_kernel_edges(pkg, oracle, gpu, ty, weighted, index, pm, out, length
 def test_any_kernel_fp8_formats(pkg, oracle, gpu, bits, bias, weighted):
     # up to 4 exponent bits codes are read as shifted fp16 halves, above through fp32
     test_any_kernel_edges(pkg, oracle, gpu, FP8, weighted, torch.int32, 0, FP32, "short", fp8=(bits, bias))
+
+
+@pytest.mark.parametrize("out,D", [(FP32, 16), (FP16, 64), (BF16, 128), (FP16, 144), (FP32, 1040), (FP16, 2064)])
+@pytest.mark.parametrize("ty", sorted(PER_WORD))
+def test_nobag_batches(pkg, oracle, gpu, ty, out, D):
+    # sequence rows: segments cut inside and at the edges of the 8-load batches and 64-index
+    # chunks, widths of one load, of a cut last lane and of several column tiles
+    specs = [(60 + 9 * t, D, pkg.SparseType(ty)) for t in range(3)]
+    m = pkg.IntNBitTableBatchedEmbeddingBagsCodegen(specs, device=gpu, pooling_mode=2, output_dtype=out)
+    m.fill_random_weights(4)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(D)
+    L = torch.tensor([1, 63, 0, 64, 7, 130, 8, 9, 0, 15, 31, 1], device=gpu)
+    idx = torch.cat([torch.randint(-1, E + 1, (int(L[t * 4:t * 4 + 4].sum()),), device=gpu, generator=g)
+                     for t, (E, _, _) in enumerate(specs)]).to(torch.int32)
+    off = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), L.cumsum(0)]).to(torch.int32)
+    _check_module(oracle, m, idx, off, None, f"nobag ty={ty} D={D} out={out}")
