@@ -87,30 +87,36 @@ __device__ __forceinline__ void any_bag(const KParams& p, const TbeTableDesc& td
   for (int e = 0; e < E; ++e) acc[e] = 0.f;
   float bacc = 0.f;
 
-  // lane l < S: index l of the step at row q (zero past the bag)
-  auto load_idx = [&](int q, uint64_t& idx, float& w) __attribute__((always_inline)) {
-    const int n = uniform(max(0, min(S, L - q)));
-    const int64_t at = n > 0 ? start + q : 0;
-    idx = load_index_chunk<IndexT>(p, at, n);
-    w = WEIGHTED ? load_weight_chunk(p, at, n) : 0.f;
+  AnyStep<U, VW> regs[2];
+  uint64_t idx[2];
+  float psw[2];
+  // lane l < S: index l of the step at position `at`, `left` rows before the bag's end
+  // (zero past it)
+  auto load_idx = [&](auto set, int64_t at, int left) __attribute__((always_inline)) {
+    const int n = uniform(max(0, min(S, left)));
+    if (n == 0) at = 0;
+    idx[set()] = load_index_chunk<IndexT>(p, at, n);
+    psw[set()] = WEIGHTED ? load_weight_chunk(p, at, n) : 0.f;
   };
-  auto issue = [&](int q, uint64_t idx, float w, AnyStep<U, VW>& r) __attribute__((always_inline)) {
-    const uint32_t off = (lane < L - q && idx < rows) ? static_cast<uint32_t>(idx) * stride : kNoRow;
+  auto issue = [&](auto set, int left) __attribute__((always_inline)) {
+    AnyStep<U, VW>& r = regs[set()];
+    const uint32_t off = (lane < left && idx[set()] < rows) ? static_cast<uint32_t>(idx[set()]) * stride : kNoRow;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int src = (u * R + slot) * 4;
       const uint32_t o = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(src, static_cast<int>(off)));
       load_words<VW>(rs, o + col, r.d[u]);
       r.h[u] = HDR ? static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(o), 0, 0)) : 0u;
-      r.w[u] = WEIGHTED ? __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(w))) : 1.f;
+      r.w[u] = WEIGHTED ? __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(psw[set()]))) : 1.f;
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto consume = [&](int q, const AnyStep<U, VW>& r) __attribute__((always_inline)) {
+  auto consume = [&](auto set, int left) __attribute__((always_inline)) {
+    const AnyStep<U, VW>& r = regs[set()];
     constexpr bool kPair = !WEIGHTED && kPairDot<WT>;
 #pragma unroll
     for (int u = 0; u < U; u += kPair ? 2 : 1) {
-      if (q + u * R >= L) break;  // wave-uniform
+      if (u * R >= left) break;  // wave-uniform
 #pragma unroll
       for (int v = 0; v < VW; ++v) {  // the row's bias once, with its first word
         float unused = 0.f;
@@ -122,27 +128,7 @@ __device__ __forceinline__ void any_bag(const KParams& p, const TbeTableDesc& td
       }
     }
   };
-
-  if (L > 0) {
-    AnyStep<U, VW> ra, rb;
-    uint64_t i0, i1;
-    float w0, w1;
-    load_idx(0, i0, w0);
-    load_idx(S, i1, w1);
-    issue(0, i0, w0, ra);
-    for (int q = 0;;) {
-      load_idx(q + 2 * S, i0, w0);
-      issue(q + S, i1, w1, rb);
-      consume(q, ra);
-      q += S;
-      if (q >= L) break;
-      load_idx(q + 2 * S, i1, w1);
-      issue(q + S, i0, w0, ra);
-      consume(q, rb);
-      q += S;
-      if (q >= L) break;
-    }
-  }
+  if (L > 0) walk_steps(start, L, S, load_idx, issue, consume);
 
   if constexpr (VW == 1 || kHalf) reduce_slots<E, HDR>(acc, bacc, lg);
   if constexpr (WPB > 1) {
@@ -218,10 +204,9 @@ __global__ __launch_bounds__(kBlock) void pooled_any_kernel(KParams p) {
   const int len = uniform(static_cast<int>(end - start));
   int L = len;
   if constexpr (WPB > 1) {  // this wave's share of the rows
-    const int per = (len + WPB - 1) / WPB;
-    const int first = min(wv * per, len);
-    start += first;
-    L = min(per, len - first);
+    const BagShare share = bag_share(len, wv, WPB);
+    start += share.first;
+    L = share.rows;
   }
   switch (td.weight_ty) {
     case TBE_TY_INT4: any_table<TBE_TY_INT4, WEIGHTED, WPB, IndexT>(p, td, start, L, len, ct, b, sh); break;

@@ -57,6 +57,7 @@
 #include <utility>
 #include <vector>
 
+#include "tbe_bag_walk.h"
 #include "tbe_internal.h"
 #include "tbe_nbit.h"
 namespace tbe {
@@ -1013,17 +1014,16 @@ __device__ __forceinline__ void finish_bag_fast(const KParams& p, const StagedBa
   const int n0 = min(L, kWave);
   consume_step<WT, LG, WEIGHTED, VW>(p, r0, 0, n0, acc, bacc);
   pool_steps<WT, LG, WEIGHTED, VW, A64>(p, c, my_off, sb.w, n0, 1, acc, bacc);
-  for (int base = kWave; base < L; base += kWave) {
-    const int n = min(kWave, L - base);
-    const uint64_t idx = load_index_chunk<IndexT>(p, sb.start + base, n);
-    const float w = WEIGHTED ? load_weight_chunk(p, sb.start + base, n) : 0.f;
+  walk_chunks(sb.start + kWave, L - kWave, kWave, [&](int64_t at, int n) __attribute__((always_inline)) {
+    const uint64_t idx = load_index_chunk<IndexT>(p, at, n);
+    const float w = WEIGHTED ? load_weight_chunk(p, at, n) : 0.f;
     const uint32_t off = row_offset<A64>(c, idx, n);
     StepRegs<unroll_for<LG, VW>(), VW> r;
     issue_step<WT, LG, WEIGHTED, VW, A64>(c, off, w, 0, r);
     __builtin_amdgcn_sched_barrier(0);
     consume_step<WT, LG, WEIGHTED, VW>(p, r, 0, n, acc, bacc);
     pool_steps<WT, LG, WEIGHTED, VW, A64>(p, c, off, w, n, 1, acc, bacc);
-  }
+  });
   if (sb.valid) reduce_store<WT, LG, E>(p, c.td, L, c.dw, c.col_ok, sb.b, acc, bacc);
 }
 
@@ -1053,14 +1053,13 @@ __device__ __forceinline__ void pool_bag_wide(const KParams& p, const TbeTableDe
   for (int e = 0; e < E; ++e) acc[e] = 0.f;
   float bacc = 0.f;
 
-  for (int base = 0; base < L; base += kWave) {
-    const int n = min(kWave, L - base);
+  walk_chunks(start, L, kWave, [&](int64_t at, int n) __attribute__((always_inline)) {
     int64_t my_row = -1;
     float my_w = 0.f;
     if (lane < n) {
-      const int64_t idx = load_index(p, p.indices, start + base + lane);
+      const int64_t idx = load_index(p, p.indices, at + lane);
       if (idx >= 0 && idx < rows) my_row = idx;
-      if constexpr (WEIGHTED) my_w = p.psw[start + base + lane];
+      if constexpr (WEIGHTED) my_w = p.psw[at + lane];
     }
     const int32_t row_lo = static_cast<int32_t>(my_row);
     const int32_t row_hi = static_cast<int32_t>(my_row >> 32);
@@ -1092,7 +1091,7 @@ __device__ __forceinline__ void pool_bag_wide(const KParams& p, const TbeTableDe
       for (int u = 0; u < kUnrollWide; ++u)
         if (r0 + u * R < n) accum_row<WT, WEIGHTED>(acc, bacc, d[u], h[u], w[u], p.fp8);
     }
-  }
+  });
 
   reduce_slots<E, HDR>(acc, bacc, lg);
   if (slot == 0 && col_ok) finish_bag<WT>(p, td, L, dw, b, acc, bacc);
