@@ -14,9 +14,10 @@ import numpy as np
 from . import HIP_LIB
 
 ABI_VERSION = 3
-EXPORTS = ("tbe_nbit_plan", "tbe_nbit_forward", "tbe_last_error", "tbe_nbit_abi_version",
+EXPORTS = ("tbe_nbit_plan", "tbe_nbit_forward", "tbe_nbit_pooled_kernels", "tbe_last_error", "tbe_nbit_abi_version",
            "tbe_permute_pooled_embs", "tbe_block_bucketize_workspace_bytes",
-           "tbe_block_bucketize_store_lists", "tbe_block_bucketize_sparse_features", "tbe_block_bucketize_sparse_features_noalloc")
+           "tbe_block_bucketize_store_lists", "tbe_block_bucketize_sparse_features",
+           "tbe_block_bucketize_sparse_features_noalloc")
 # TBE_BLOCK_BUCKETIZE_NOALLOC_SCRATCH_BYTES of include/tbe_sparse_ops.h
 NOALLOC_SCRATCH_BYTES = 32 << 20
 
@@ -26,6 +27,7 @@ TBE_FLAG_NO_STREAM = 0x2
 TBE_FLAG_FORCE_STREAM = 0x4
 TBE_FLAG_SERIAL_GROUPS = 0x8
 TBE_FLAG_NARROW_WORDS = 0x10
+TBE_POOLED_BAG, TBE_POOLED_STREAM, TBE_POOLED_ANY, TBE_POOLED_ONE = range(4)  # TbePooledKernel
 TBE_TABLE_OFFSET32 = 0x1
 TBE_TABLE_STREAM = 0x2
 
@@ -119,6 +121,8 @@ def lib():
                                     ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(TbePlanSummary)]
         L.tbe_nbit_forward.restype = ctypes.c_int
         L.tbe_nbit_forward.argtypes = [ctypes.POINTER(TbeNbitArgs), ctypes.c_void_p]
+        L.tbe_nbit_pooled_kernels.restype = ctypes.c_int
+        L.tbe_nbit_pooled_kernels.argtypes = [ctypes.POINTER(TbeNbitArgs), ctypes.POINTER(ctypes.c_int32)]
         L.tbe_last_error.restype = ctypes.c_char_p
         L.tbe_last_error.argtypes = []
         L.tbe_nbit_abi_version.restype = ctypes.c_int
@@ -174,6 +178,21 @@ def forward(args: TbeNbitArgs, stream: int = 0) -> None:
     rc = lib().tbe_nbit_forward(ctypes.byref(args), ctypes.c_void_p(stream))
     if rc != TBE_OK:
         raise TbeError(rc, last_error())
+
+
+def pooled_kernels(summary: TbePlanSummary, T: int, B: int, num_indices: int, weighted: bool = False,
+                   output_dtype: int = 0, flags: int = 0):
+    """The TBE_POOLED_* kernel of each table group of a pooled call of these sizes."""
+    a = TbeNbitArgs()
+    a.plan = ctypes.pointer(summary)
+    a.T, a.B, a.num_indices, a.max_col_tiles = T, B, num_indices, summary.max_col_tiles
+    a.indice_weights = 1 if weighted else None  # only asked whether there are any
+    a.output_dtype, a.flags = int(output_dtype), int(flags)
+    kinds = (ctypes.c_int32 * TBE_MAX_GROUPS)()
+    rc = lib().tbe_nbit_pooled_kernels(ctypes.byref(a), kinds)
+    if rc != TBE_OK:
+        raise TbeError(rc, last_error())
+    return list(kinds[:summary.num_groups])
 
 
 def forward_tensors(dev_weights, weights_offsets, weights_tys, D_offsets, indices, offsets,

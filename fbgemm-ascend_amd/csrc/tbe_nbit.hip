@@ -280,6 +280,14 @@ KernelFn pooled_kernel_for(const TbePlanGroup& g, bool index64, bool weighted, b
   }
 }
 
+// A launch holds fewer than 2^32 threads.  The any-type kernel takes a wave (split: a
+// work-group) per item and is not persistent, so past this its groups go to the others.
+constexpr int64_t kMaxBlocks = 0xFFFFFFFFLL / kBlock;
+
+int64_t any_blocks(int64_t items, bool split) {
+  return split ? items : (items + kWavesPerBlock - 1) / kWavesPerBlock;
+}
+
 // Calls of several table groups with at most this many bags take the one kernel for
 // every type and width (tbe_kern_any.hip) instead of a launch per group: 15 launches of
 // 5 us kernels cost ~95 us whatever the batch.  64 mixed tables (weighted mean, 32 rows
@@ -290,6 +298,14 @@ constexpr int64_t kAnyMaxBags = int64_t(1) << 17;
 
 // the flags that choose a kernel per group keep doing so
 constexpr int32_t kKernelFlags = TBE_FLAG_NO_STREAM | TBE_FLAG_FORCE_STREAM | TBE_FLAG_NARROW_WORDS;
+
+// Column tiles of the one launch: those of the widest table.
+int any_call_tiles(const TbePlanSummary& plan) {
+  int tiles = 1;
+  for (int gi = 0; gi < plan.num_groups; ++gi)
+    tiles = std::max(tiles, any_col_tiles(plan.groups[gi].weight_ty, plan.groups[gi].col_tiles));
+  return tiles;
+}
 
 bool use_any_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan) {
   if (a->flags & kKernelFlags) return false;
@@ -323,7 +339,7 @@ bool use_any_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan) {
 //    of 32 rows: 789 -> 832 us; of 5 rows, with the row streams above: 486 -> 399).
 enum class Pool { kBag, kStream, kAny };
 
-Pool pick_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const TbePlanGroup& g, int64_t rows_per_bag) {
+Pool preferred_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const TbePlanGroup& g, int64_t rows_per_bag) {
   if (!g.offset32 || a->num_indices > 0x7FFFFFFF) return Pool::kBag;
   const bool stream = g.stream && !(a->flags & TBE_FLAG_NO_STREAM);
   const bool many = static_cast<int64_t>(g.count) * a->B * g.col_tiles >= kStreamMinBags;
@@ -348,6 +364,14 @@ Pool pick_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const TbePlan
       rows_per_bag >= kAnyRowsPerBag * (a->indice_weights ? 2 : 1))
     return Pool::kAny;
   return Pool::kBag;
+}
+
+Pool pick_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const TbePlanGroup& g, int64_t rows_per_bag) {
+  const Pool k = preferred_kernel(a, plan, g, rows_per_bag);
+  if (k != Pool::kAny ||
+      any_blocks(static_cast<int64_t>(g.count) * a->B * any_col_tiles(g.weight_ty, g.col_tiles), false) <= kMaxBlocks)
+    return k;
+  return g.stream ? Pool::kStream : Pool::kBag;
 }
 
 // Four waves per bag instead of one when bags are long and too few to fill the GPU
@@ -457,7 +481,18 @@ hipError_t launch_any(KParams& p, int64_t items, int tiles, bool weighted, bool 
   p.div_tiles = make_fastdiv(static_cast<uint32_t>(tiles));
   p.num_items = static_cast<int32_t>(items);
   return launch(any_kernel(p.index64 != 0, weighted, split), p,
-                split ? items : (items + kWavesPerBlock - 1) / kWavesPerBlock, false, s);
+                any_blocks(items, split), false, s);
+}
+
+// The checks of a plan's groups that the launches rely on.
+int check_plan(const TbeNbitArgs* a, const TbePlanSummary& plan) {
+  if (plan.num_groups < 1 || plan.num_groups > TBE_MAX_GROUPS) return fail(TBE_ERR_INVALID_ARG, "bad plan");
+  for (int gi = 0; gi < plan.num_groups; ++gi) {
+    const TbePlanGroup& g = plan.groups[gi];
+    if (g.count <= 0 || g.first < 0 || g.first + g.count > a->T || g.col_tiles < 1 || g.col_tiles > 255)
+      return fail(TBE_ERR_INVALID_ARG, "bad plan group %d", gi);
+  }
+  return TBE_OK;
 }
 
 }  // namespace tbe
@@ -594,6 +629,23 @@ int tbe_nbit_plan(const TbePlanInput* in, TbeTableDesc* descs, int32_t* table_or
   return TBE_OK;
 }
 
+int tbe_nbit_pooled_kernels(const TbeNbitArgs* a, int32_t* kinds) {
+  g_last_error.clear();
+  if (!a || !a->plan || !kinds) return fail(TBE_ERR_INVALID_ARG, "null argument to tbe_nbit_pooled_kernels");
+  if (a->T <= 0 || a->B <= 0 || a->num_indices < 0) return fail(TBE_ERR_INVALID_ARG, "no bags");
+  if (check_plan(a, *a->plan) != TBE_OK) return TBE_ERR_INVALID_ARG;
+  const bool one = use_any_kernel(a, *a->plan);
+  const int64_t rows_per_bag = a->num_indices / (static_cast<int64_t>(a->T) * a->B);
+  for (int gi = 0; gi < a->plan->num_groups; ++gi) {
+    const Pool k = one ? Pool::kAny : pick_kernel(a, *a->plan, a->plan->groups[gi], rows_per_bag);
+    kinds[gi] = one                  ? TBE_POOLED_ONE
+                : k == Pool::kAny    ? TBE_POOLED_ANY
+                : k == Pool::kStream ? TBE_POOLED_STREAM
+                                     : TBE_POOLED_BAG;
+  }
+  return TBE_OK;
+}
+
 int tbe_nbit_forward(const TbeNbitArgs* a, void* hip_stream) {
   g_last_error.clear();
   if (!a) return fail(TBE_ERR_INVALID_ARG, "null args");
@@ -672,20 +724,13 @@ int tbe_nbit_forward(const TbeNbitArgs* a, void* hip_stream) {
 
   if (!a->table_order) return fail(TBE_ERR_INVALID_ARG, "null table_order");
   const TbePlanSummary& plan = *a->plan;
-  if (plan.num_groups < 1 || plan.num_groups > TBE_MAX_GROUPS) return fail(TBE_ERR_INVALID_ARG, "bad plan");
-  for (int gi = 0; gi < plan.num_groups; ++gi) {
-    const TbePlanGroup& g = plan.groups[gi];
-    if (g.count <= 0 || g.first < 0 || g.first + g.count > a->T || g.col_tiles < 1 || g.col_tiles > 255)
-      return fail(TBE_ERR_INVALID_ARG, "bad plan group %d", gi);
-  }
+  if (check_plan(a, plan) != TBE_OK) return TBE_ERR_INVALID_ARG;
   const bool weighted = a->indice_weights != nullptr;
   // the per-group kernels keep index positions in 32 bits
   const bool wide = a->num_indices > 0x7FFFFFFF;
   const int64_t rows_per_bag = a->num_indices / nbags;
   if (use_any_kernel(a, plan)) {
-    int tiles = 1;
-    for (int gi = 0; gi < plan.num_groups; ++gi)
-      tiles = std::max(tiles, any_col_tiles(plan.groups[gi].weight_ty, plan.groups[gi].col_tiles));
+    const int tiles = any_call_tiles(plan);
     p.order = nullptr;
     const hipError_t err =
         launch_any(p, nbags * tiles, tiles, weighted, any_split(nbags * tiles, rows_per_bag), s);

@@ -186,6 +186,21 @@ int tbe_nbit_plan(const TbePlanInput* in, TbeTableDesc* descs, int32_t* table_or
  */
 int tbe_nbit_forward(const TbeNbitArgs* args, void* hip_stream);
 
+/* The kernels of a pooled call. */
+enum TbePooledKernel {
+  TBE_POOLED_BAG = 0,     /* a wave per bag, persistent                              */
+  TBE_POOLED_STREAM = 1,  /* slots of lanes walk index runs across bags              */
+  TBE_POOLED_ANY = 2,     /* the any-type kernel, one launch for the group           */
+  TBE_POOLED_ONE = 3      /* the any-type kernel, one launch for every group         */
+};
+
+/*
+ * The TbePooledKernel that tbe_nbit_forward takes for each table group of a pooled
+ * call: kinds[plan->num_groups].  Reads the sizes, the flags, the plan and whether
+ * weights are given; no device memory, no launch.
+ */
+int tbe_nbit_pooled_kernels(const TbeNbitArgs* args, int32_t* kinds);
+
 /* Message of the last failure on the calling thread ("" if none). */
 const char* tbe_last_error(void);
 
