@@ -6,12 +6,11 @@
 //   PK = src/pooled_embedding_ops/permute_pooled_embs/v220/op_kernel/permute_pooled_embs_kernel.h
 //
 // permute_pooled_embs is a strided column copy: HBM-bound, 2 * B * total_D *
-// elem_size bytes per call.  A thread owns one 16-byte chunk of the output's columns and
-// copies it row by row, so stores are contiguous whatever the segments' widths.  Where the
-// chunk's bytes come from is found once per thread from the three device lists, which the
-// host never reads (the reference reads offset_dim_list[T] on the host, PA:82): mostly one
-// run of the input row (one 16-byte load), else two (two loads merged under a byte mask),
-// else element by element (segments of a few bytes).  Loads and stores need no alignment.
+// elem_size bytes per call.  One work-group copies one segment (a feature's columns) for a
+// block of rows; the segment's source/destination columns come from the three device
+// lists, so the host never reads them (the reference reads offset_dim_list[T] on the host,
+// PA:82).  Consecutive lanes take consecutive 16-byte vectors of a row, at any alignment
+// where the segment is 16 bytes or wider.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -27,13 +26,10 @@ namespace tbe {
 namespace {
 
 constexpr int kPermBlock = 256;
-constexpr int kPermRows = 64;      // most rows of one work-group
-constexpr int kPermUnroll = 4;     // rows a thread has in flight
-constexpr int kPermLdsLists = 2048;  // segments whose starts are kept in LDS
-constexpr int64_t kPermGroups = 2048;
-constexpr int64_t kPermNarrowRow = 2560;
-constexpr int32_t kPermZero = -1;  // unit of a segment without a source: zero
-constexpr int32_t kPermSkip = -2;  // byte outside every segment: not written
+constexpr int kPermRows = 64;       // most rows of one work-group
+constexpr int64_t kPermChunks = 264;  // 16-byte vectors of a work-group, at the mean segment width
+constexpr int kPermXcds = 8;
+constexpr int64_t kPermMaxBlocks = 0xFFFFFFFFLL / kPermBlock;  // a launch holds fewer than 2^32 threads
 
 struct PermParams {
   const uint8_t* __restrict__ in;
@@ -43,14 +39,11 @@ struct PermParams {
   const int64_t* __restrict__ inv;
   int64_t B;
   int64_t total_D;
-  int64_t col_bytes;    // bytes of one column of one row (inner * elem_size)
+  int64_t col_bytes;   // bytes of one column of one row (inner * elem_size)
   int32_t T;
-  int32_t row_bytes;
-  int32_t col_blocks;   // work-groups side by side over a row
-  int32_t chunks;       // chunks of a row a work-group covers
-  int32_t row_step;     // rows it covers at a time
-  int32_t rows;         // rows of one work-group
-  int32_t seg_blocks;   // segment kernel: work-groups per segment
+  int32_t rows;        // rows of one work-group
+  int32_t row_blocks;  // work-groups per segment
+  int32_t grouped;     // 1: the work-groups of one row block share an XCD
 };
 
 struct Vec16 {
@@ -94,7 +87,7 @@ __device__ __forceinline__ void copy_rows(const PermParams& p, int64_t r0, int64
                                           int64_t nbytes, bool zero) {
   using V = typename std::conditional<VB == 16, uint4,
             typename std::conditional<VB == 4, uint32_t, uint16_t>::type>::type;
-  const int64_t row_bytes = p.row_bytes;
+  const int64_t row_bytes = p.total_D * p.col_bytes;
   const uint32_t nv = static_cast<uint32_t>(nbytes / VB);
   if (nv == 0) return;
   const uint32_t items = static_cast<uint32_t>(r1 - r0) * nv;
@@ -112,16 +105,53 @@ __device__ __forceinline__ void copy_rows(const PermParams& p, int64_t r0, int64
   }
 }
 
-// Rows of at most kPermNarrowRow bytes: a work-group copies one segment (PK:173-211) for
-// kPermRows rows (PK:140-170) with 16-, 4- or 2-byte vectors by alignment.  It finds its
-// columns with three loads and leaves no thread idle at the row's end: 12 segments of
-// 64-128 fp16 columns, 16384 rows 16.9 us against 20.4 by chunks, 10 of 1-31 columns 5.6
-// against 8.7.
+// The same at any alignment, for 16 bytes or more per row: the last vector of a row ends
+// with it and overlaps the one before.
+__device__ __forceinline__ void copy_rows_unaligned(const PermParams& p, int64_t r0, int64_t r1, int64_t src,
+                                                    int64_t dst, int64_t nbytes, bool zero) {
+  const int64_t row_bytes = p.total_D * p.col_bytes;
+  const uint32_t nv = static_cast<uint32_t>((nbytes + 15) / 16);
+  const uint32_t last = static_cast<uint32_t>(nbytes) - 16;
+  const uint32_t items = static_cast<uint32_t>(r1 - r0) * nv;
+  const UDiv div(nv);
+#pragma unroll 2
+  for (uint32_t it = threadIdx.x; it < items; it += kPermBlock) {
+    const uint32_t r = div(it);
+    const int64_t at = (r0 + r) * row_bytes + min((it - r * nv) * 16, last);
+    store16(p.out + at + dst, zero ? Vec16{} : load16(p.in + at + src));
+  }
+}
+
+// Bound by HBM traffic: one segment (PK:173-211) for a block of rows (PK:140-170).
+//  * A work-group takes the power of two of rows, at most 64, that gives it 264 to 528
+//    vectors of a mean segment.  More leave the segments of a row further apart in time, so
+//    that the lines two of them share are read and written back twice; fewer do not pay for
+//    the work-group.  Tensors in HBM in turn, 4 / 8 / 16 / 32 / 64 rows: [8192, 5864] fp16,
+//    64 segments of 8-256 columns 131 / 75 / 47 / 47 / 56 us; [1024, 19136] fp32, 200 of
+//    64-128 columns 54 / 34 / 30 / 33 / 35.
+//  * The work-groups of a row block go to one XCD, one after another (the hardware deals
+//    them round robin), so that those shared lines meet in its L2: [16384, 16000] fp16,
+//    1000 of 16 columns 463 -> 272 us.  With fewer row blocks than XCDs, row blocks run side
+//    by side and segments one after another ([256, 27512] fp16, 1000 segments of 4-60
+//    columns: 9.7 us; the other way round 12.7).
+//  * Segments that are not 16-byte aligned are copied with unaligned 16-byte vectors, not
+//    with the 4 or 2 bytes that all of their addresses are multiples of.
+// Against one work-group per 64 rows with aligned vectors only, fp16: 64 segments of 8-256
+// columns, 8192 rows 70 -> 47 us; 200 of 128, 4096 rows 88 -> 74; 1 of 4096, 4096 rows 75 ->
+// 14.
 __global__ __launch_bounds__(kPermBlock) void permute_segments_kernel(PermParams p) {
-  const int seg = static_cast<int>(blockIdx.x / static_cast<uint32_t>(p.seg_blocks));
-  const int rb = static_cast<int>(blockIdx.x - static_cast<uint32_t>(seg) * static_cast<uint32_t>(p.seg_blocks));
-  const int64_t r0 = static_cast<int64_t>(rb) * kPermRows;
-  const int64_t r1 = std::min<int64_t>(r0 + kPermRows, p.B);
+  uint32_t seg, rb;
+  if (p.grouped) {
+    const uint32_t k = blockIdx.x / kPermXcds, T = static_cast<uint32_t>(p.T);
+    rb = k / T * kPermXcds + blockIdx.x % kPermXcds;
+    seg = k % T;
+    if (rb >= static_cast<uint32_t>(p.row_blocks)) return;
+  } else {
+    seg = blockIdx.x / static_cast<uint32_t>(p.row_blocks);
+    rb = blockIdx.x % static_cast<uint32_t>(p.row_blocks);
+  }
+  const int64_t r0 = static_cast<int64_t>(rb) * p.rows;
+  const int64_t r1 = std::min<int64_t>(r0 + p.rows, p.B);
   const int64_t pi = uniform_load(p.perm + seg);
   const int64_t dst = uniform_load(p.inv + seg);
   const int64_t dst_end = uniform_load(p.inv + seg + 1);
@@ -138,172 +168,13 @@ __global__ __launch_bounds__(kPermBlock) void permute_segments_kernel(PermParams
   const uintptr_t base = reinterpret_cast<uintptr_t>(p.in) | reinterpret_cast<uintptr_t>(p.out);
   if (((sb | db | nb | rowb | static_cast<int64_t>(base)) & 15) == 0) {
     copy_rows<16>(p, r0, r1, sb, db, nb, zero);
+  } else if (nb >= 16) {
+    copy_rows_unaligned(p, r0, r1, sb, db, nb, zero);
   } else if (((sb | db | nb | rowb | static_cast<int64_t>(base)) & 3) == 0) {
     copy_rows<4>(p, r0, r1, sb, db, nb, zero);
   } else {
     // 2-byte elements (or, for misaligned fp32 buffers, half-words)
     copy_rows<2>(p, r0, r1, sb, db, nb, zero);
-  }
-}
-
-// Source byte in the input row of the columns segment `seg` copies (kPermZero: none),
-// PK:173-211.
-__device__ __forceinline__ int32_t perm_source(const PermParams& p, int seg, int64_t len_cols) {
-  const int64_t pi = p.perm[seg];
-  if (pi < 0 || pi >= p.T) return kPermZero;
-  const int64_t src = p.off[pi];
-  return src < 0 || src + len_cols > p.total_D ? kPermZero : static_cast<int32_t>(src * p.col_bytes);
-}
-
-// Lists whose segments do not follow one another (no valid call): segment after segment, in
-// list order, as far as each lies in the row.
-template <int ES>
-__device__ void perm_by_segment(const PermParams& p, int64_t r0, int64_t r1) {
-  using E = typename std::conditional<ES == 2, uint16_t, uint32_t>::type;
-  for (int seg = 0; seg < p.T; ++seg) {
-    const int64_t dst = p.inv[seg], len = p.inv[seg + 1] - dst;
-    if (dst < 0 || len < 0 || dst + len > p.total_D) continue;
-    const int32_t src = perm_source(p, seg, len);
-    const int64_t n = len * p.col_bytes / ES;
-    for (int64_t r = r0; r < r1; ++r) {
-      uint8_t* o = p.out + r * p.row_bytes + dst * p.col_bytes;
-      const uint8_t* i = p.in + r * p.row_bytes + (src < 0 ? 0 : src);
-      for (int64_t k = threadIdx.x; k < n; k += blockDim.x) {
-        E v = 0;
-        if (src >= 0) __builtin_memcpy(&v, i + k * ES, ES);
-        __builtin_memcpy(o + k * ES, &v, ES);
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// Bound by HBM traffic.  [8192, 5856] fp16, 64 segments of 8-256 columns (8-byte aligned):
-// 63.5 -> 46.3 us in HBM (1.5 GB of tensors in turn; the copy's own time 38.3); the same in
-// fp32 54.7 -> 43.8; 64 of 4-60 columns, 16384 rows 44.8 -> 29.9; 200 of 128 columns 170.5
-// -> 165.0.  Copied a segment at a time, rows of odd widths share lines between
-// work-groups on different XCDs, which read and write back each such line twice.
-template <int ES>
-__global__ __launch_bounds__(kPermBlock) void permute_pooled_kernel(PermParams p) {
-  using E = typename std::conditional<ES == 2, uint16_t, uint32_t>::type;
-  constexpr int U = 16 / ES;  // units of a chunk
-  __shared__ int32_t starts[kPermLdsLists + 1];
-  __shared__ int32_t sources[kPermLdsLists];
-  const uint32_t cb = blockIdx.x % static_cast<uint32_t>(p.col_blocks);
-  const int64_t r0 = static_cast<int64_t>(blockIdx.x / static_cast<uint32_t>(p.col_blocks)) * p.rows;
-  const int64_t r1 = std::min<int64_t>(r0 + p.rows, p.B);
-  const bool in_lds = p.T <= kPermLdsLists;
-  bool bad = false;
-  for (int i = threadIdx.x; i <= p.T; i += blockDim.x) {
-    const int64_t v = p.inv[i], next = i < p.T ? p.inv[i + 1] : v;
-    bad |= v < 0 || v > p.total_D || next < v;
-    if (in_lds) {
-      starts[i] = static_cast<int32_t>(v * p.col_bytes);
-      if (i < p.T) sources[i] = perm_source(p, i, next - v);
-    }
-  }
-  if (__syncthreads_or(bad)) {
-    if (cb == 0) perm_by_segment<ES>(p, r0, r1);
-    return;
-  }
-  auto start_of = [&](int s) { return in_lds ? starts[s] : static_cast<int32_t>(p.inv[s] * p.col_bytes); };
-  auto source_of = [&](int s) { return in_lds ? sources[s] : perm_source(p, s, p.inv[s + 1] - p.inv[s]); };
-
-  const int ty = static_cast<int>(threadIdx.x / static_cast<uint32_t>(p.chunks));
-  const int x = (static_cast<int>(cb) * p.chunks + static_cast<int>(threadIdx.x) - ty * p.chunks) * 16;
-  if (x >= p.row_bytes || ty >= p.row_step) return;
-  // last segment starting at or before x
-  int s = 0, hi = p.T - 1;
-  while (s < hi) {
-    const int mid = (s + hi + 1) >> 1;
-    if (start_of(mid) <= x) s = mid; else hi = mid - 1;
-  }
-  int32_t at[U];  // source byte of every unit
-  {
-    int begin = start_of(s), end = start_of(s + 1);
-    int32_t src = source_of(s);
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      const int y = x + j * ES;
-      while (y >= end && s + 1 < p.T) {
-        ++s;
-        begin = end;
-        end = start_of(s + 1);
-        if (y < end) src = source_of(s);
-      }
-      at[j] = y >= p.row_bytes || y < begin || y >= end ? kPermSkip : src < 0 ? kPermZero : src + (y - begin);
-    }
-  }
-  // one run, or a run and a second one from unit `cut` on (a chunk from its would-be start `b`)
-  int cut = U;
-#pragma unroll
-  for (int j = U - 1; j > 0; --j)
-    if (at[j] != at[0] + j * ES) cut = j;
-  int b = 0;
-  uint32_t m[4] = {0, 0, 0, 0};  // bytes of the second run
-  bool runs = at[0] >= 0, whole = at[0] != kPermSkip;  // every byte has a source / is written
-#pragma unroll
-  for (int j = 1; j < U; ++j) {
-    if (j == cut) b = at[j] - j * ES;
-    whole = whole && at[j] != kPermSkip;
-    runs = runs && at[j] >= 0 && (j < cut || at[j] == b + j * ES);
-    if (j >= cut) m[j * ES / 4] |= ES == 4 ? 0xFFFFFFFFu : 0xFFFFu << (16 * (j & 1));
-  }
-  const bool two = cut < U;
-  const int step = p.row_step;
-  for (int64_t r = r0 + ty; r < r1; r += kPermUnroll * step) {
-    // both loads of a two-run chunk reach past their segment: not in the tensor's first
-    // and last row
-    if (runs && !(two && (r == 0 || r + (kPermUnroll - 1) * static_cast<int64_t>(step) >= p.B - 1))) {
-      Vec16 v[kPermUnroll], w[kPermUnroll];
-#pragma unroll
-      for (int i = 0; i < kPermUnroll; ++i) {
-        const int64_t row = r + i * step;
-        if (row < r1) {
-          const uint8_t* q = p.in + row * p.row_bytes;
-          v[i] = load16(q + at[0]);
-          if (two) w[i] = load16(q + b);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < kPermUnroll; ++i) {
-        const int64_t row = r + i * step;
-        if (row < r1) {
-          if (two) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[i].w[k] = (v[i].w[k] & ~m[k]) | (w[i].w[k] & m[k]);
-          }
-          store16(p.out + row * p.row_bytes + x, v[i]);
-        }
-      }
-    } else {
-      E e[kPermUnroll][U];
-#pragma unroll
-      for (int i = 0; i < kPermUnroll; ++i) {
-        const int64_t row = std::min<int64_t>(r + i * step, r1 - 1);
-        const uint8_t* q = p.in + row * p.row_bytes;
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-          e[i][j] = 0;
-          if (at[j] >= 0) __builtin_memcpy(&e[i][j], q + at[j], ES);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < kPermUnroll; ++i) {
-        const int64_t row = r + i * step;
-        if (row >= r1) break;
-        uint8_t* o = p.out + row * p.row_bytes + x;
-        if (whole) {
-          Vec16 v;
-          __builtin_memcpy(&v, e[i], 16);
-          store16(o, v);
-        } else {
-#pragma unroll
-          for (int j = 0; j < U; ++j)
-            if (at[j] != kPermSkip) __builtin_memcpy(o + j * ES, &e[i][j], ES);
-        }
-      }
-    }
   }
 }
 
@@ -326,32 +197,6 @@ extern "C" int tbe_permute_pooled_embs(const TbePermutePooledArgs* a, void* hip_
   const int64_t row_bytes = a->total_D * a->inner * a->elem_size;
   if ((a->B + kPermRows - 1) / kPermRows * a->T > 0x7FFFFFFF || row_bytes * kPermRows > 0x7FFFFFFF)
     return fail(TBE_ERR_UNSUPPORTED, "permute_pooled_embs shape too large for one launch");
-  // A work-group covers whole rows where they fit its 256 threads (as many at a time as
-  // leave the fewest threads of its waves idle), else an even share of up to 256 chunks.
-  // Narrower shares lose more to partial lines than idle threads cost: rows of 88 chunks,
-  // one at a time by 128 threads of 256 14.3 us, as 3 x 32 chunks 18.4.
-  const int64_t chunks = (row_bytes + 15) / 16;
-  const int64_t col_blocks = (chunks + kPermBlock - 1) / kPermBlock;
-  int cw = static_cast<int>((chunks + col_blocks - 1) / col_blocks);
-  if (col_blocks > 1) cw = (cw + 15) / 16 * 16;  // shares of whole 128-byte lines
-  int row_step = 1, threads = 0;
-  for (int k = 1; k * cw <= kPermBlock; ++k) {
-    const int t = (k * cw + 63) / 64 * 64;
-    if (threads == 0 || k * cw * threads >= row_step * cw * t) {
-      row_step = k;
-      threads = t;
-    }
-  }
-  // about kPermGroups work-groups of whole unrolled steps (a work-group finds its columns'
-  // sources first: [512, 5856] fp16 in 1536 of one row 12.1 us, in 384 of four 8.8), or of
-  // whole steps where one covers several narrow rows (10 features, 16384 rows: 256 of 64
-  // rows 11.3 us, 910 of 18 rows 8.7)
-  const int64_t unit = row_step < kPermUnroll ? row_step * kPermUnroll : row_step;
-  int64_t rows = std::min<int64_t>((a->B * col_blocks + kPermGroups - 1) / kPermGroups, kPermRows);
-  rows = (rows + unit - 1) / unit * unit;
-  const int64_t row_blocks = (a->B + rows - 1) / rows;
-  if (row_blocks * col_blocks > 0x7FFFFFFF)
-    return fail(TBE_ERR_UNSUPPORTED, "permute_pooled_embs shape too large for one launch");
   PermParams p{};
   p.in = static_cast<const uint8_t*>(a->pooled_embs);
   p.out = static_cast<uint8_t*>(a->output);
@@ -362,21 +207,28 @@ extern "C" int tbe_permute_pooled_embs(const TbePermutePooledArgs* a, void* hip_
   p.total_D = a->total_D;
   p.col_bytes = a->inner * a->elem_size;
   p.T = a->T;
-  p.row_bytes = static_cast<int32_t>(row_bytes);
-  p.col_blocks = static_cast<int32_t>(col_blocks);
-  p.chunks = cw;
-  p.row_step = row_step;
-  p.rows = static_cast<int32_t>(rows);
-  p.seg_blocks = static_cast<int32_t>((a->B + kPermRows - 1) / kPermRows);
-  const bool narrow = row_bytes <= kPermNarrowRow;
-  const void* fn = narrow              ? reinterpret_cast<const void*>(permute_segments_kernel)
-                   : a->elem_size == 2 ? reinterpret_cast<const void*>(permute_pooled_kernel<2>)
-                                       : reinterpret_cast<const void*>(permute_pooled_kernel<4>);
-  const int64_t blocks = narrow ? static_cast<int64_t>(p.seg_blocks) * a->T : row_blocks * col_blocks;
+  int64_t rows = kPermRows;
+  while (rows > 1 && rows / 2 * row_bytes >= kPermChunks * 16 * a->T) rows /= 2;
+  auto groups = [&] {
+    p.rows = static_cast<int32_t>(rows);
+    p.row_blocks = static_cast<int32_t>((a->B + rows - 1) / rows);
+    p.grouped = p.row_blocks >= kPermXcds;
+    const int64_t rb = p.row_blocks;
+    return (p.grouped ? (rb + kPermXcds - 1) / kPermXcds * kPermXcds : rb) * a->T;
+  };
+  int64_t blocks = groups();
+  while (blocks > kPermMaxBlocks && rows < kPermRows) {
+    rows *= 2;
+    blocks = groups();
+  }
+  if (blocks > kPermMaxBlocks && p.grouped) {  // no room for the last group's padding
+    p.grouped = 0;
+    blocks = static_cast<int64_t>(p.row_blocks) * a->T;
+  }
   void* args[] = {&p};
-  const hipError_t err = hipLaunchKernel(fn, dim3(static_cast<uint32_t>(blocks)),
-                                         dim3(static_cast<uint32_t>(narrow ? kPermBlock : threads)), args, 0,
-                                         static_cast<hipStream_t>(hip_stream));
+  const hipError_t err =
+      hipLaunchKernel(reinterpret_cast<const void*>(permute_segments_kernel), dim3(static_cast<uint32_t>(blocks)),
+                      dim3(kPermBlock), args, 0, static_cast<hipStream_t>(hip_stream));
   if (err != hipSuccess) return fail(TBE_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
   return TBE_OK;
 }
