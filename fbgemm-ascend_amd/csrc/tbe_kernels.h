@@ -1561,7 +1561,9 @@ __device__ __forceinline__ void nobag_segment(const KParams& p, const TbeTableDe
   const uint32_t off = A64 ? (has_row ? static_cast<uint32_t>(iv) : kNoRow64)
                            : (has_row ? static_cast<uint32_t>(iv) * stride : kNoRow);
   const uint8_t* tbase = p.weights + td.weights_offset;
-  const bool vec = (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0 && p.out_stride % E == 0;
+  // range-checked vector stores: the bytes of 64 output rows have to fit 32 bits
+  const bool vec = (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0 && p.out_stride % E == 0 &&
+                   p.out_stride < (int64_t(1) << 24);
   const uint32_t es = p.out_ty == TBE_TY_FP32 ? 4u : 2u;
   const uint32_t out_row = static_cast<uint32_t>(uniform(static_cast<int>(static_cast<uint32_t>(p.out_stride) * es)));
   const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(

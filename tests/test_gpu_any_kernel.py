@@ -59,3 +59,22 @@ def test_nobag_batches(pkg, oracle, gpu, ty, out, D):
                      for t, (E, _, _) in enumerate(specs)]).to(torch.int32)
     off = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), L.cumsum(0)]).to(torch.int32)
     _check_module(oracle, m, idx, off, None, f"nobag ty={ty} D={D} out={out}")
+
+
+@pytest.mark.parametrize("ty,out", [(INT8, FP32), (FP16, FP16), (INT4, BF16)])
+def test_nobag_far_output_rows(pkg, gpu, ty, out):
+    # output rows so far apart that 64 of them span more than 4 GiB
+    D = 16 * PER_WORD[ty] if ty != INT4 else 32 * PER_WORD[ty]
+    m = pkg.IntNBitTableBatchedEmbeddingBagsCodegen([(50, D, pkg.SparseType(ty))], device=gpu, pooling_mode=2,
+                                                    output_dtype=out)
+    m.fill_random_weights(4)
+    idx = torch.arange(-1, 65, dtype=torch.int32, device=gpu)  # -1 and 50 on: zero rows
+    off = torch.tensor([0, idx.numel()], dtype=torch.int32, device=gpu)
+    want = m(idx, off, None)
+    stride = ((1 << 32) // (64 * want.element_size())) + 16
+    far = torch.empty((idx.numel(), stride), dtype=want.dtype, device=gpu)
+    far[:, :D] = 7
+    print(f"[gpu] nobag far rows ty={ty} stride={stride}", flush=True)
+    pkg.capi.forward_tensors(m.weights_dev, m.weights_offsets, m.weights_tys, m.D_offsets, idx, off, 2, None,
+                             m.output_dtype, m.row_alignment, out=far)
+    assert torch.equal(far[:, :D], want)
