@@ -544,7 +544,7 @@ __global__ __launch_bounds__(kBBBlock) void bb_count(BBParams<IT, OT> p) {
 template <typename IT>
 struct ScatterStage {
   IT v[kChunk * kWaveBB];         // new index of each slot
-  uint32_t meta[kChunk * kWaveBB];  // bucket | (position in the chunk << 8)
+  uint16_t meta[kChunk * kWaveBB];  // bucket | (position in the chunk << 6)
   int64_t cur[kWaveBB];           // row's next output offset per bucket
   int64_t delta[kWaveBB];         // output offset - slot, per bucket, this chunk
   uint32_t cnt[kWaveBB];          // chunk count, then next slot, per bucket
@@ -564,11 +564,11 @@ __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t x) {
 // ONLY_FAST (rows marked fast): gives up on the row, returning false, at the
 // first chunk holding an index at or above gsize, before writing anything of that
 // chunk; the general pass then rewrites the whole row (the same values at the same
-// positions).  Returns true when the row is done.  `cur`: the row's first output offset
-// per bucket where the caller holds it, instead of p.new_offsets.
-template <bool FAST, int NB, typename IT, typename OT, bool ONLY_FAST = false>
+// positions).  Returns true when the row is done.  HAVE_CUR: st.cur holds the row's first
+// output offset per bucket already.
+template <bool FAST, int NB, typename IT, typename OT, bool ONLY_FAST = false, bool HAVE_CUR = false>
 __device__ __forceinline__ bool scatter_row_staged(const BBParams<IT, OT>& p, const RowCtx<IT>& c, int64_t r,
-                                                   ScatterStage<IT>& st, const int64_t* cur = nullptr) {
+                                                   ScatterStage<IT>& st) {
   using UIT = std::make_unsigned_t<IT>;
   constexpr uint32_t kNone = 0xFFu;
   const UIT* __restrict__ idx = reinterpret_cast<const UIT*>(p.indices);
@@ -579,8 +579,7 @@ __device__ __forceinline__ bool scatter_row_staged(const BBParams<IT, OT>& p, co
     for (int k = 0; k < kChunk; ++k)  // clamped, not branched: the row is not empty
       uk[k] = idx[std::min<int64_t>(chunk + k * kWaveBB + lane, c.e - 1)];
     // the row's cursors, loaded with its first indices (one wait for both)
-    if (chunk == c.s && lane < p.my_size)
-      st.cur[lane] = cur ? cur[lane] : static_cast<int64_t>(p.new_offsets[lane * p.L + r]);
+    if (!HAVE_CUR && chunk == c.s && lane < p.my_size) st.cur[lane] = static_cast<int64_t>(p.new_offsets[lane * p.L + r]);
     if constexpr (ONLY_FAST) {
       bool high = false;
 #pragma unroll
@@ -626,7 +625,7 @@ __device__ __forceinline__ bool scatter_row_staged(const BBParams<IT, OT>& p, co
                                                                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mine), 0u));
         if ((mine >> lane) == 1) st.cnt[bk[k]] = slot + 1;
         st.v[slot] = vk[k];
-        st.meta[slot] = bk[k] | (static_cast<uint32_t>(k * kWaveBB + lane) << 8);
+        st.meta[slot] = static_cast<uint16_t>(bk[k] | (static_cast<uint32_t>(k * kWaveBB + lane) << 6));
       }
     }
     // 4. write out in slot order
@@ -634,8 +633,8 @@ __device__ __forceinline__ bool scatter_row_staged(const BBParams<IT, OT>& p, co
       const uint32_t t = t0 + static_cast<uint32_t>(lane);
       if (t < total) {
         const uint32_t m = st.meta[t];
-        const int64_t w = st.delta[m & 0xFFu] + t;
-        const int64_t i = chunk + (m >> 8);
+        const int64_t w = st.delta[m & 0x3Fu] + t;
+        const int64_t i = chunk + (m >> 6);
         if (w >= 0 && w < p.N) {
           p.new_indices[w] = st.v[t];
           if (p.new_weights) p.new_weights[w] = p.weights[i];
@@ -757,9 +756,9 @@ __global__ __launch_bounds__(kBBBlock) void bb_scatter(BBParams<IT, OT> p) {
 // Phase 2: out[0] = 0, out[k + 1] = in[0] + ... + in[k] over n elements, in three
 // passes: tile sums, an exclusive scan of the tile sums by one work-group, then
 // each tile's scan plus its base.
-template <typename T>
+template <int WAVES = kBBBlock / kWaveBB, typename T>
 __device__ __forceinline__ T block_exclusive_scan(T v, T* lds_wave, T& total) {
-  // inclusive scan inside the wave with DPP-free shuffles, then across the 4 waves
+  // inclusive scan inside the wave with DPP-free shuffles, then across the waves
   const int lane = lane_id();
   T x = v;
 #pragma unroll
@@ -772,7 +771,7 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* lds_wave, T& total) {
   __syncthreads();
   T wbase = 0;
   total = 0;
-  for (int k = 0; k < kBBBlock / kWaveBB; ++k) {
+  for (int k = 0; k < WAVES; ++k) {
     if (k < w) wbase += lds_wave[k];
     total += lds_wave[k];
   }
@@ -880,35 +879,36 @@ __global__ __launch_bounds__(kBBBlock) void scan_tiles_based(const T* __restrict
 // a work-group of the count sums the lengths before its rows itself, and a work-group of
 // the scatter sums the bucket totals that the count's work-groups left (my_size x groups
 // values, from L2) instead of scanning my_size x L counts.  48 features x 32 rows, 12 ranks
-// (37 k weighted int64 indices): 28.2 -> 15.9 us.
+// (37 k weighted int64 indices): 28.2 -> 14.7 us.
 
-constexpr int kFewRowsMax = 16;  // rows of one work-group
+// A work-group has a wave per row (W of both), as the general path deals them: with 2 or 4
+// consecutive rows a wave, a feature of long rows was left to a few waves (96 features x 128
+// rows, 737 k int32 indices, 90 % of them in one feature: 224 us, the general path 77, now 95).
 
-template <typename IT, typename OT>
-__global__ __launch_bounds__(kBBBlock) void bb_count_few(BBParams<IT, OT> p, const OT* __restrict__ lengths,
-                                                        OT* __restrict__ formed, OT* __restrict__ sums, int per) {
-  __shared__ uint32_t lds_hist[kBBBlock / kWaveBB][kWaveBB];
+template <typename IT, typename OT, int W>
+__global__ __launch_bounds__(W * kWaveBB) void bb_count_few(BBParams<IT, OT> p, const OT* __restrict__ lengths,
+                                                           OT* __restrict__ formed, OT* __restrict__ sums) {
+  __shared__ uint32_t lds_hist[W][kWaveBB];
   __shared__ uint32_t group_sum[kWaveBB];
-  __shared__ OT own[kFewRowsMax + 1];
-  __shared__ OT lds_wave[kBBBlock / kWaveBB];
-  constexpr int kWaves = kBBBlock / kWaveBB;
+  __shared__ OT own[W + 1];
+  __shared__ OT lds_wave[W];
   const int lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   uint32_t* hist = lds_hist[wv];
   hist[lane] = 0;
   if (wv == 0) group_sum[lane] = 0;
-  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * per;
-  const int n = static_cast<int>(std::min<int64_t>(per, p.L - b0));
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * W;
+  const int n = static_cast<int>(std::min<int64_t>(W, p.L - b0));
   if (lengths) {
     OT part = 0;
 #pragma unroll 4
-    for (int64_t r = threadIdx.x; r < b0; r += kBBBlock) part += lengths[r];
+    for (int64_t r = threadIdx.x; r < b0; r += W * kWaveBB) part += lengths[r];
     OT base;
-    (void)block_exclusive_scan(part, lds_wave, base);
+    (void)block_exclusive_scan<W>(part, lds_wave, base);
     if (wv == 0) {
       OT x = lane < n ? lengths[b0 + lane] : OT(0);
 #pragma unroll
-      for (int d = 1; d < kFewRowsMax; d <<= 1) {
+      for (int d = 1; d < W; d <<= 1) {
         const OT y = __shfl_up(x, d, kWaveBB);
         if (lane >= d) x += y;
       }
@@ -923,18 +923,14 @@ __global__ __launch_bounds__(kBBBlock) void bb_count_few(BBParams<IT, OT> p, con
     }
   }
   __syncthreads();
-  // this wave's rows: b0 + wv, then every kWaves-th
-  const int mine_i = wv + lane * kWaves;
-  const RowCtx<IT> mine = row_ctx_lane(p, mine_i < n ? b0 + mine_i : -1, lengths ? own : nullptr, b0);
-  for (int j = 0; wv + j * kWaves < n; ++j) {
-    const int64_t r = b0 + wv + j * kWaves;
-    const RowCtx<IT> c = row_ctx_of(mine, j);
+  if (wv < n) {  // wave-uniform
+    const int64_t r = b0 + wv;
+    const RowCtx<IT> c = row_ctx_of(row_ctx_lane(p, r, lengths ? own : nullptr, b0), 0);
     if (c.ok) {
       if (c.fast) count_row<true, true>(p, c, r, hist, nullptr);
       else count_row<false, true>(p, c, r, hist, nullptr);
     }
     const uint32_t cnt = hist[lane];  // the wave's LDS operations complete in order
-    hist[lane] = 0;
     if (lane < p.my_size) p.new_lengths[lane * p.L + r] = static_cast<OT>(cnt);
     atomicAdd(group_sum + lane, cnt);
   }
@@ -942,27 +938,24 @@ __global__ __launch_bounds__(kBBBlock) void bb_count_few(BBParams<IT, OT> p, con
   if (wv == 0 && lane < p.my_size) sums[static_cast<int64_t>(lane) * gridDim.x + blockIdx.x] = static_cast<OT>(group_sum[lane]);
 }
 
-template <typename IT, typename OT, int NB>
-__global__ __launch_bounds__(kBBBlock) void bb_scatter_few(BBParams<IT, OT> p, const OT* __restrict__ sums, int per) {
-  __shared__ ScatterStage<IT> lds_stage[kBBBlock / kWaveBB];
-  __shared__ int64_t cur[kFewRowsMax][kWaveBB];
+template <typename IT, typename OT, int NB, int W>
+__global__ __launch_bounds__(W * kWaveBB) void bb_scatter_few(BBParams<IT, OT> p, const OT* __restrict__ sums) {
+  __shared__ ScatterStage<IT> lds_stage[W];
   __shared__ OT total[kWaveBB], before[kWaveBB];  // per bucket: all rows, and the rows before this group's
-  constexpr int kWaves = kBBBlock / kWaveBB;
   const int lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   ScatterStage<IT>& st = lds_stage[wv];
   st.cnt[lane] = 0;
   const int my = static_cast<int>(p.my_size);
-  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * per;
-  const int n = static_cast<int>(std::min<int64_t>(per, p.L - b0));
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * W;
+  const int n = static_cast<int>(std::min<int64_t>(W, p.L - b0));
   // what the rows need besides the totals loads first, behind the sums below
-  const int mine_i = wv + lane * kWaves;
-  const RowCtx<IT> mine = row_ctx_lane(p, mine_i < n ? b0 + mine_i : -1);
-  OT cnt[kFewRowsMax];
+  const RowCtx<IT> mine = row_ctx_lane(p, wv < n ? b0 + wv : -1);
+  OT cnt[W];
 #pragma unroll
-  for (int i = 0; i < kFewRowsMax; ++i)
+  for (int i = 0; i < W; ++i)
     cnt[i] = wv == 0 && i < n && lane < my ? p.new_lengths[lane * p.L + b0 + i] : OT(0);
-  for (int b = wv; b < my; b += kWaves) {
+  for (int b = wv; b < my; b += W) {
     OT all = 0, pre = 0;
 #pragma unroll 4
     for (uint32_t i = lane; i < gridDim.x; i += kWaveBB) {
@@ -993,9 +986,9 @@ __global__ __launch_bounds__(kBBBlock) void bb_scatter_few(BBParams<IT, OT> p, c
       OT run = x - own + before[lane];
       OT* out = const_cast<OT*>(p.new_offsets) + lane * p.L + b0;
 #pragma unroll
-      for (int i = 0; i < kFewRowsMax; ++i) {
+      for (int i = 0; i < W; ++i) {
         if (i >= n) break;
-        cur[i][lane] = static_cast<int64_t>(run);
+        lds_stage[i].cur[lane] = static_cast<int64_t>(run);
         out[i] = run;
         run += cnt[i];
       }
@@ -1003,29 +996,41 @@ __global__ __launch_bounds__(kBBBlock) void bb_scatter_few(BBParams<IT, OT> p, c
     }
   }
   __syncthreads();
-  for (int j = 0; wv + j * kWaves < n; ++j) {
-    const int i = wv + j * kWaves;
-    const RowCtx<IT> c = row_ctx_of(mine, j);
-    if (!c.ok) continue;
-    if (c.fast) scatter_row_staged<true, NB>(p, c, b0 + i, st, cur[i]);
-    else scatter_row_staged<false, NB>(p, c, b0 + i, st, cur[i]);
-  }
+  const RowCtx<IT> c = row_ctx_of(mine, 0);
+  if (!c.ok) return;  // wave-uniform, past the last barrier
+  if (c.fast) scatter_row_staged<true, NB, IT, OT, false, true>(p, c, b0 + wv, st);
+  else scatter_row_staged<false, NB, IT, OT, false, true>(p, c, b0 + wv, st);
 }
 
-// Rows per work-group of the two launches, 0 where the general path is used.  The lines:
-// a work-group reads at most 16 k lengths and 16 k bucket totals, one row per wave while
-// the totals stay below 8 k (1536 rows, 12 ranks: 4 rows a group 15.9 us, 8 rows 17.4, 16
-// rows 21.8; 12288 rows, 8 ranks: 8 rows 47.3, 16 rows 44.6); past a million indices the general scatter's fast pass (more
-// waves per SIMD) is worth its launches (8192 rows, int64, 16 ranks: 2.6 M indices 43.8 us
-// against 45.6 in two launches; 12288 rows, 8 ranks, 983 k int32: 42.1 against 30.4), four
-// million with bucket boundaries, which the fast pass does not take.
+// Rows (and waves) per work-group of the two launches, 0 where the general path is used.
+// The lines (us as general / two launches; int64, rows of 30 indices unless said):
+//  * A work-group reads all lengths before its rows and all bucket totals: fewer, larger ones
+//    from 2048 and 4096 rows and past 8 k totals (3328 rows, 16 ranks: 8 rows a group 27 /
+//    17, 16 rows 21).  Past 32 ranks 16 waves share the totals' sums (1536 rows, 64 ranks:
+//    27 / 20; 4 rows a group 34).
+//  * 16 waves of int64 indices fill a CU's LDS, and all wait for the sums: 8192 rows, 8
+//    ranks 35 / 27, 12288 rows 42 / 40, but with 90 % of the indices in one of 96 features
+//    57 / 66.  int32 (two groups a CU): 12288 rows 38 / 31 and 53 / 58, 16384 rows 44 / 39
+//    and 50 / 55.
+//  * Past a million indices the general scatter's fast pass, of more waves per SIMD, is worth
+//    its launches (8192 rows, 16 ranks, 2.6 M indices 43.8 / 45.6).  Bucket boundaries keep
+//    rows from it: four million (12288 rows, 8 ranks, 737 k int32 49 / 39).
 constexpr int64_t kFewIndices = int64_t(1) << 20;
 
-int few_rows_per_group(int64_t my, int64_t L, int64_t N, bool lists) {
-  if (my > kWaveBB || L < 1 || L > 16384 || N > (lists ? 4 : 1) * kFewIndices) return 0;
-  for (int per = 4; per <= kFewRowsMax; per *= 2)
-    if ((L + per - 1) / per * my <= (per < kFewRowsMax ? 8192 : 16384)) return per;
+int few_rows_per_group(int64_t my, int64_t L, int64_t N, bool lists, int32_t index_size) {
+  if (my > kWaveBB || L < 1 || N > (lists ? 4 : 1) * kFewIndices) return 0;
+  if (L > (lists || index_size == 4 ? 12288 : 8192)) return 0;
+  for (int per = my > 32 || L > 4096 ? 16 : L > 2048 ? 8 : 4; per <= 16; per *= 2)
+    if ((L + per - 1) / per * my <= (per < 16 ? 8192 : 16384)) return per;
   return 0;
+}
+
+template <typename IT, typename OT, int W>
+void launch_few(const BBParams<IT, OT>& p, const OT* lengths, OT* formed, OT* sums, bool few_buckets, hipStream_t s) {
+  const dim3 g(static_cast<uint32_t>((p.L + W - 1) / W)), b(W * kWaveBB);
+  hipLaunchKernelGGL((bb_count_few<IT, OT, W>), g, b, 0, s, p, lengths, formed, sums);
+  if (few_buckets) hipLaunchKernelGGL((bb_scatter_few<IT, OT, 4, W>), g, b, 0, s, p, const_cast<const OT*>(sums));
+  else hipLaunchKernelGGL((bb_scatter_few<IT, OT, 6, W>), g, b, 0, s, p, const_cast<const OT*>(sums));
 }
 
 int64_t scan_tiles_of(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
@@ -1135,18 +1140,15 @@ int run(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_of
   p.keep = a->keep_orig_idx;
   int nbits = 0;  // ceil(log2(my_size))
   while (nbits < 6 && (int64_t(1) << nbits) < a->my_size) ++nbits;
-  const int per = few_rows_per_group(a->my_size, p.L, p.N, p.pos != nullptr);
+  const int per = few_rows_per_group(a->my_size, p.L, p.N, p.pos != nullptr, a->index_size);
   if (per > 0) {
     const int64_t groups = (p.L + per - 1) / per;
     if (groups * a->my_size * static_cast<int64_t>(sizeof(OT)) <= few_bytes) {
       OT* group_sums = static_cast<OT*>(few_sums);
-      const dim3 g(static_cast<uint32_t>(groups));
-      hipLaunchKernelGGL((bb_count_few<IT, OT>), g, dim3(kBBBlock), 0, s, p,
-                         a->offsets ? nullptr : static_cast<const OT*>(a->lengths), formed, group_sums, per);
-      if (nbits <= 4)
-        hipLaunchKernelGGL((bb_scatter_few<IT, OT, 4>), g, dim3(kBBBlock), 0, s, p, const_cast<const OT*>(group_sums), per);
-      else
-        hipLaunchKernelGGL((bb_scatter_few<IT, OT, 6>), g, dim3(kBBBlock), 0, s, p, const_cast<const OT*>(group_sums), per);
+      const OT* lengths = a->offsets ? nullptr : static_cast<const OT*>(a->lengths);
+      if (per == 4) launch_few<IT, OT, 4>(p, lengths, formed, group_sums, nbits <= 4, s);
+      else if (per == 8) launch_few<IT, OT, 8>(p, lengths, formed, group_sums, nbits <= 4, s);
+      else launch_few<IT, OT, 16>(p, lengths, formed, group_sums, nbits <= 4, s);
       const hipError_t err = hipGetLastError();
       if (err != hipSuccess) return fail(TBE_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
       return TBE_OK;

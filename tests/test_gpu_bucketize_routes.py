@@ -60,6 +60,17 @@ def test_few_rows(pkg, oracle, gpu, F, B, my, dtype, lists):
     _compare(oracle, gpu, lengths, indices, np.full(F, 25, dtype), my, pos)
 
 
+# a wave per row in groups of 4, 8 and 16 rows: the lines between them, and the last rows
+# taken without and with lists (8192 of int64, 12288)
+@pytest.mark.parametrize("F,B,my,dtype", [
+    (1, 2048, 2, np.int64), (1, 2049, 2, np.int64), (1, 4095, 16, np.int32), (1, 4096, 17, np.int64),
+    (1, 4097, 2, np.int64), (3, 5, 40, np.int64), (2, 4096, 32, np.int64), (1, 8192, 33, np.int64),
+    (1, 8193, 8, np.int64), (4, 3072, 8, np.int32), (1, 12289, 8, np.int32), (3, 4095, 21, np.int64)])
+@pytest.mark.parametrize("lists", [False, True])
+def test_few_rows_groups(pkg, oracle, gpu, F, B, my, dtype, lists):
+    test_few_rows(pkg, oracle, gpu, F, B, my, dtype, lists)
+
+
 @pytest.mark.parametrize("L", [1, 5, 4099])
 def test_few_rows_c_abi(pkg, oracle, gpu, L):
     # offsets given or formed, scratch of the caller or the library's own; new_offsets is an output
