@@ -207,7 +207,6 @@ KernelFn stream_kernel_group(const TbePlanGroup& g, bool index64, bool weighted,
 // kernel whatever their rows per bag; smaller ones as pick_kernel says.
 constexpr int64_t kStreamMinBags = int64_t(1) << 20;
 constexpr int64_t kStreamBagsPerRow = 49152;
-constexpr int64_t kAnyRowsPerBag = 24;
 
 // Rows a wave of the row-stream kernel should walk: measured on 200 INT4 tables x
 // 32768 bags of ~40 rows, 32 bags per wave (1280 rows) ran 3.14 ms, 24 or 40 bags
@@ -288,13 +287,24 @@ int64_t any_blocks(int64_t items, bool split) {
   return split ? items : (items + kWavesPerBlock - 1) / kWavesPerBlock;
 }
 
-// Calls of several table groups with at most this many bags take the one kernel for
-// every type and width (tbe_kern_any.hip) instead of a launch per group: 15 launches of
-// 5 us kernels cost ~95 us whatever the batch.  64 mixed tables (weighted mean, 32 rows
-// a bag): 2 k bags 93 -> 7 us, 32 k bags 95 -> 32, 128 k bags 156 -> 113, 524 k bags
-// 461 -> 516.  The line is at half of the crossing because short
-// bags cross earlier (its waves take ~0.5 ns a bag however short, the others ~0.2).
+// Calls of several table groups take the one kernel for every type and width
+// (tbe_kern_any.hip) instead of a launch per group while it costs less than the launches.
+// us, a launch per group / one launch:
+//  * Launches: ~40 + 5 a group where the host sets the pace (2 groups 48, 3 groups 54, 6
+//    groups 70, 12 groups 96), ~10 + 4 a group from a captured graph.
+//  * The one launch: 0.4-0.55 ns a wave however short its bag, 0.2 ns a wave without work
+//    (every table gets the column tiles of the widest).  Two groups (INT8 and INT4 D 64), 2
+//    rows a bag: 32 k bags 47 / 16, 65 k 47 / 28 (23 / 28 captured), 131 k 52 / 58; 12
+//    groups: 131 k bags 97 / 61 (59 / 61 captured).  45 tables of 64 columns and 3 of 4096
+//    (16 tiles), 16 k bags: 48 / 59, 131 k bags: 76 / 450.
+//    The line: 0.25 ns a wave, twice that with work, against 24 us + 5 a group.
+//  * Long bags cost the same in either, and waves ending with their bag save more: 131 k
+//    bags of 60 rows 93 / 82 (2 groups), 135 / 101 (12 groups); 64 mixed tables, 32 rows a
+//    bag: 128 k bags 156 / 113, 524 k 461 / 516.  Up to 2^17 waves, and short bags too.
 constexpr int64_t kAnyMaxBags = int64_t(1) << 17;
+constexpr int64_t kAnyWaves = 96 << 10;          // 24 us of waves without work
+constexpr int64_t kAnyWavesPerGroup = 20 << 10;  // 5 us
+constexpr int64_t kAnyRowsPerBag = 24;           // long bags, here and in preferred_kernel
 
 // the flags that choose a kernel per group keep doing so
 constexpr int32_t kKernelFlags = TBE_FLAG_NO_STREAM | TBE_FLAG_FORCE_STREAM | TBE_FLAG_NARROW_WORDS;
@@ -309,11 +319,17 @@ int any_call_tiles(const TbePlanSummary& plan) {
 
 bool use_any_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan) {
   if (a->flags & kKernelFlags) return false;
-  if (plan.num_groups < 2 || a->num_indices > 0x7FFFFFFF || static_cast<int64_t>(a->T) * a->B > kAnyMaxBags)
-    return false;
-  for (int gi = 0; gi < plan.num_groups; ++gi)  // 32-bit row offsets only
-    if (!plan.groups[gi].offset32) return false;
-  return true;
+  if (plan.num_groups < 2 || a->num_indices > 0x7FFFFFFF) return false;
+  int64_t busy = 0;  // waves with work
+  for (int gi = 0; gi < plan.num_groups; ++gi) {
+    const TbePlanGroup& g = plan.groups[gi];
+    if (!g.offset32) return false;  // 32-bit row offsets only
+    busy += static_cast<int64_t>(g.count) * a->B * any_col_tiles(g.weight_ty, g.col_tiles);
+  }
+  const int64_t bags = static_cast<int64_t>(a->T) * a->B;
+  const int64_t waves = bags * any_call_tiles(plan);
+  if (a->num_indices >= bags * kAnyRowsPerBag) return waves <= kAnyMaxBags;
+  return bags <= kAnyMaxBags && waves + busy <= kAnyWaves + kAnyWavesPerGroup * plan.num_groups;
 }
 
 // The kernel of one group: per-bag, row-stream or the any-type kernel, by the group's

@@ -21,6 +21,9 @@ pytestmark = pytest.mark.gpu
     ((INT8,), 64, 1, 49151, 1, False), ((INT4,), 64, 1, 49152, 1, True),       # 49152 bags per row of a bag
     ((INT8, FP16, FP32), 128, 3, 43690, 1, False), ((INT8, FP16, FP32), 128, 3, 43691, 1, False),  # 2^17 bags in all
     ((INT2, BF16), 64, 2, 65537, 2, True),
+    ((INT8, FP16, FP32), 128, 3, 26624, 2, True), ((INT8, FP16, FP32), 128, 3, 26625, 2, True),  # short bags, 3 groups
+    ((INT8, FP16, FP32), 128, 3, 43690, 24, False),                            # long bags: 2^17 in all
+    ((INT2, FP8), 1024, 2, 65537, 9, True),    # past both: the any-type kernel for the second group alone
 ])
 def test_dispatch_lines(pkg, oracle, gpu, types, D, T, B, rows, weighted):
     specs = [(500 + 30 * t, D, pkg.SparseType(types[t % len(types)])) for t in range(T)]

@@ -27,3 +27,25 @@ def test_launch_fits_the_grid(pkg, ty, D, rows):
     for B in (most - 3, most + 1, 0x7FFFFFFF // tiles):
         for k in kinds(pkg, [(1000, D, ty)], B, rows):
             assert k in (c.TBE_POOLED_BAG, c.TBE_POOLED_STREAM) or (k == c.TBE_POOLED_ANY and B <= most), B
+
+
+NARROW2 = [(1000, 64, INT8), (1000, 64, INT4)]
+NARROW12 = [(1000, D, ty) for ty in (INT8, INT4, INT2, FP16) for D in (32, 64, 128)]
+
+
+@pytest.mark.parametrize("specs,bags,rows,one", [
+    # short bags: the waves of one launch against the launches it saves
+    (NARROW2 * 8, 69_632, 2, True), (NARROW2 * 8, 69_648, 2, False), (NARROW2 * 8, 131_072, 23, False),
+    (NARROW12 * 4, 131_040, 2, True),
+    # long bags
+    (NARROW2 * 8, 131_072, 24, True), (NARROW2 * 8, 131_088, 24, False), (NARROW12 * 4, 131_136, 60, False),
+    # every table gets the column tiles of the widest: 16
+    (NARROW2 * 7 + [(1000, 4096, FP32)], 16_384, 2, False), (NARROW2 * 7 + [(1000, 4096, FP32)], 4_096, 2, True),
+    (NARROW2 * 7 + [(1000, 4096, FP32)], 8_175, 40, True), (NARROW2 * 7 + [(1000, 4096, FP32)], 16_384, 40, False),
+])
+def test_one_launch_of_several_groups(pkg, specs, bags, rows, one):
+    c = pkg.capi
+    got = kinds(pkg, specs, bags // len(specs), rows)
+    assert all((k == c.TBE_POOLED_ONE) == one for k in got), got
+    flagged = kinds(pkg, specs, bags // len(specs), rows, flags=c.TBE_FLAG_NO_STREAM)
+    assert c.TBE_POOLED_ONE not in flagged and c.TBE_POOLED_ANY not in flagged
