@@ -334,25 +334,34 @@ bool use_any_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan) {
 
 // The kernel of one group: per-bag, row-stream or the any-type kernel, by the group's
 // bags, rows per bag and row width.  The lines lie where 16 tables of that shape crossed
-// (Zipf 1.05; us as per-bag / row-stream / any):
+// (Zipf 1.05, fp16 out; us as per-bag / the other):
 //  * Row streams share a wave's set-up among its bags, so they win where bags are short
 //    and many.  Rows up to 32 words: from ~49 k bags per row of a bag (INT8 D 64, 524 k
-//    bags: 2 rows 93 / 42, 5 rows 106 / 66, 12 rows 122 / 109, 30 rows 207 / 214; 131 k
-//    bags: 2 rows 28 / 24, 5 rows 29 / 29), and always from 2^20 bags x column tiles.
-//  * Rows of 33-128 words, plain float: FP32 D 128, 8 k bags: 12 rows 12 / 10 / 11, 30
-//    rows 17 / 17 / 16; 131 k bags: 5 rows 82 / 39 / 75, 30 rows 220 / 189 / 208, 60 rows
-//    392 / 350 / 347.  INT8 and FP8 rows, which cost more to decode: INT8 D 512, 8 k bags:
-//    5 rows 12 / 11 / 11; 32 k bags: 5 rows 29 / 24 / 28, 12 rows 41 / 37 / 39, 30 rows
-//    84 / 83 / 78; 131 k bags: 12 rows 163 / 136 / 175, 30 rows 301 / 265 / 284.
-//  * Rows past 128 words: the any kernel reads 256 words of a row at a time (FP8 D 1024,
-//    32 k bags: 5 rows 53 / 42 / 32, 30 rows 154 / 129 / 100; FP32 D 512: 30 rows 234 /
-//    200 / 153), all but the shortest plain-float bags (131 k bags, 2 rows 267 / 85 / 153).
-//  * Else rows of 33 words or more take the any kernel from about 24 rows a bag, where its
-//    waves ending with their bag beats the persistent pipeline (INT8 D 256, 32 k bags: 5
-//    rows 17 / 16 / 19, 30 rows 42 / 44 / 38, 60 rows 78 / 84 / 67).  INT2 rows keep one
-//    word per lane in it (16 sums a word) and gain nothing.  Not beside other groups of
-//    a large call, whose persistent kernels its waves crowd out (64 mixed tables, 1 M bags
-//    of 32 rows: 789 -> 832 us; of 5 rows, with the row streams above: 486 -> 399).
+//    bags: 2 rows 93 / 42, 5 rows 106 / 66, 30 rows 207 / 214; 131 k bags: 2 rows 28 / 24,
+//    5 rows 29 / 29), and always from 2^20 bags x column tiles.
+//  * Rows of 33-128 words, plain float: FP32 D 128, 8 k bags: 5 rows 7.2 / 6.4, 12 rows
+//    8.2 / 8.8; 131 k bags: 12 rows 74 / 63, 24 rows 120 / 137.  INT8 and FP8 rows, which
+//    cost more to decode: INT8 D 256, 32 k bags: 2 rows 10.8 / 9.8, 5 rows 12.0 / 12.9;
+//    131 k bags: 5 rows 33 / 30, 12 rows 48 / 54; D 512, 131 k bags, 5 rows 63 / 71.
+//    INT4 and INT2 rows of 512 columns or more, whose sums fill the registers: INT4 D 512,
+//    262 k bags: 1 row 61 / 114, 2 rows 65 / 101, 5 rows 83 / 76; INT2 D 512: 79 / 111, 90 /
+//    72; INT4 D 1024, 131 k bags, 2 rows 66 / 136; INT2 D 1024, 262 k bags, 5 rows 191 / 300.
+//  * The any-type kernel's waves end with their bag, which pays while the bags are about a
+//    round of the GPU's waves; below that a long bag's serial steps are longer in it.  Rows
+//    of 33 words or more, 24 rows or more (or two tiles): FP16 D 128, 100 rows: 2 k bags
+//    9.0 / 8.5, 8 k 19.3 / 20.5; FP32 D 128, 30 rows: 4 k bags 7.8 / 8.5, 32 k 33 / 43;
+//    INT8 D 512, 60 rows: 512 bags 6.5 / 6.6, 2 k 10.8 / 10.6, 4 k 15.4 / 17.4, 32 k 99 /
+//    114.  FP8: D 256, 60 rows, 16 k bags 31 / 28, 30 rows, 32 k bags 30 / 31; D 512, 30
+//    rows, 32 k bags 53 / 50, 131 k bags 208 / 217.  INT4 D 512: 8 k bags, 30 rows 12.8 /
+//    13.5, 16 k bags, 60 rows 35 / 32, 131 k bags, 30 rows 125 / 134.  INT2 rows keep one
+//    word per lane in it (16 sums a word) and gain nothing.
+//  * Rows past 128 words: it reads 256 words of a row at a time (FP32 D 512: 8 k bags, 5
+//    rows 17 / 13, 12 rows 21 / 21, 30 rows 36 / 42; 16 k bags, 30 rows 82 / 76; D 256: 2 k
+//    bags, 16 rows 6.3 / 5.1, 16 k bags, 30 rows 34 / 38, 32 k bags 75 / 67; INT8 D 1024, 30 rows: 4 k bags 16 / 17, 16 k
+//    49 / 47; FP8 D 1024: 8 k bags, 30 rows 30 / 29; 512 bags 6.0 / 7.6), all but the shortest
+//    plain-float bags (131 k bags, 2 rows 267 / 85 as row streams / 153).
+//  * Else not beside other groups of a large call, whose persistent kernels its waves crowd
+//    out (64 mixed tables, 1 M bags of 32 rows: 789 -> 832 us).
 enum class Pool { kBag, kStream, kAny };
 
 Pool preferred_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const TbePlanGroup& g, int64_t rows_per_bag) {
@@ -363,23 +372,33 @@ Pool preferred_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const Tb
     return stream && (many || (a->flags & TBE_FLAG_FORCE_STREAM)) ? Pool::kStream : Pool::kBag;
   const bool alone = plan.num_groups == 1;
   const int64_t bags = static_cast<int64_t>(a->T) * a->B;  // the groups of a call share the GPU
-  const bool plain = g.weight_ty == TBE_TY_FP32 || g.weight_ty == TBE_TY_FP16 || g.weight_ty == TBE_TY_BF16;
-  const bool bytes = g.weight_ty == TBE_TY_INT8 || g.weight_ty == TBE_TY_FP8;
-  if (g.log2_lanes == 6 && (plain || bytes)) {
-    if (g.col_tiles > 2)
-      return stream && plain && rows_per_bag <= 8 && bags >= (1 << 15) ? Pool::kStream : Pool::kAny;
-    const int64_t few = plain ? (1 << 13) : (1 << 15);
-    const int64_t all = plain && g.col_tiles == 1 ? (1 << 15) : (1 << 17);
-    if (stream && (many || (bags >= few && rows_per_bag <= (plain ? 16 : 12)) ||
-                   (alone && bags >= all && rows_per_bag <= (plain ? 40 : 24))))
-      return Pool::kStream;
-    return alone && (g.col_tiles > 1 || rows_per_bag >= kAnyRowsPerBag) ? Pool::kAny : Pool::kBag;
+  const int64_t rows = rows_per_bag;
+  const bool short_bags = bags >= kStreamBagsPerRow * std::max<int64_t>(1, rows);
+  const bool int2 = g.weight_ty == TBE_TY_INT2, int4 = g.weight_ty == TBE_TY_INT4, fp8 = g.weight_ty == TBE_TY_FP8;
+  const bool plain = g.weight_ty != TBE_TY_INT8 && !fp8 && !int4 && !int2;
+  if (g.log2_lanes < 6 || int4 || int2) {
+    const bool wide = g.log2_lanes == 6 || (int2 && g.log2_lanes == 5);  // 512 columns or more
+    const bool fit = !wide || (rows >= 4 && g.col_tiles == 1 && !(int2 && g.log2_lanes == 6));
+    if (stream && (many || (short_bags && fit))) return Pool::kStream;
+    const bool any = int4 && wide && rows >= 48 && bags >= (1 << 11) && bags < (1 << 15);
+    return alone && any ? Pool::kAny : Pool::kBag;
   }
-  if (stream && (many || bags >= kStreamBagsPerRow * std::max<int64_t>(1, rows_per_bag))) return Pool::kStream;
-  if (alone && g.weight_ty == TBE_TY_INT4 && g.log2_lanes == 6 &&
-      rows_per_bag >= kAnyRowsPerBag * (a->indice_weights ? 2 : 1))
-    return Pool::kAny;
-  return Pool::kBag;
+  if (g.col_tiles > 2) {
+    if (stream && plain && rows <= 8 && bags >= (1 << 15)) return Pool::kStream;
+    const int64_t items = bags * g.col_tiles;
+    const bool serial = (plain && rows > 12 && items < (3 << 15)) || (!plain && !fp8 && rows > 16 && items < (1 << 15));
+    const bool few = (rows > 8 && bags < (1 << 10)) || (serial && (rows > 24 || items >= (1 << 14)));
+    return alone && few ? Pool::kBag : Pool::kAny;
+  }
+  const bool two = g.col_tiles == 2, most = bags >= (1 << 17);
+  const int64_t stream_rows = plain ? (most ? 12 : 8) : most && (fp8 || !two) ? 6 : 2;
+  if (stream && (many || (bags >= (plain ? 1 << 13 : 1 << 15) && rows <= stream_rows))) return Pool::kStream;
+  if (!alone || !(two || rows >= kAnyRowsPerBag)) return Pool::kBag;
+  const bool any = plain ? bags < (two && rows <= 16 ? 1 << 13 : 1 << 12)
+                   : !fp8 ? bags < (1 << 12) && (!two || bags >= (1 << 10))
+                   : two  ? bags >= (1 << 10) && bags < (rows >= kAnyRowsPerBag ? 1 << 17 : 1 << 14)
+                          : bags < (1 << 15);
+  return any ? Pool::kAny : Pool::kBag;
 }
 
 Pool pick_kernel(const TbeNbitArgs* a, const TbePlanSummary& plan, const TbePlanGroup& g, int64_t rows_per_bag) {

@@ -49,3 +49,27 @@ def test_one_launch_of_several_groups(pkg, specs, bags, rows, one):
     assert all((k == c.TBE_POOLED_ONE) == one for k in got), got
     flagged = kinds(pkg, specs, bags // len(specs), rows, flags=c.TBE_FLAG_NO_STREAM)
     assert c.TBE_POOLED_ONE not in flagged and c.TBE_POOLED_ANY not in flagged
+
+
+@pytest.mark.parametrize("ty,D,bags,rows,want", [
+    # row streams: short bags, not for rows of 512 columns of few bits
+    (INT8, 64, 49_152, 1, "STREAM"), (INT8, 64, 49_151, 1, "BAG"), (INT4, 512, 262_144, 2, "BAG"),
+    (INT4, 512, 262_144, 5, "STREAM"), (INT4, 1024, 262_144, 5, "BAG"), (INT2, 512, 524_288, 2, "BAG"),
+    (INT2, 512, 524_288, 5, "STREAM"), (INT2, 1024, 262_144, 5, "BAG"), (FP32, 64, 8192, 8, "STREAM"),
+    (FP32, 64, 8192, 9, "BAG"), (FP16, 256, 131_072, 12, "STREAM"), (FP16, 256, 131_072, 13, "BAG"),
+    (INT8, 256, 32_768, 2, "STREAM"), (INT8, 256, 32_768, 3, "BAG"), (INT8, 256, 131_072, 6, "STREAM"),
+    (INT8, 512, 131_072, 6, "BAG"), (FP8, 512, 131_072, 6, "STREAM"), (FP8, 512, 131_072, 7, "BAG"),
+    # 33-128 words: waves that end with their bag, for about a round of the GPU's waves
+    (FP16, 128, 4095, 24, "ANY"), (FP16, 128, 4096, 24, "BAG"), (FP16, 128, 2048, 23, "BAG"),
+    (FP32, 128, 8191, 16, "ANY"), (FP32, 128, 4096, 17, "BAG"), (INT8, 512, 1023, 60, "BAG"),
+    (INT8, 512, 1024, 60, "ANY"), (INT8, 512, 4096, 60, "BAG"), (FP8, 256, 32_767, 24, "ANY"),
+    (FP8, 256, 32_768, 24, "BAG"), (FP8, 512, 131_071, 24, "ANY"), (FP8, 512, 131_072, 24, "BAG"),
+    (INT4, 512, 2048, 48, "ANY"), (INT4, 512, 32_768, 48, "BAG"), (INT4, 512, 2048, 47, "BAG"),
+    # past 128 words: not long bags that are few
+    (FP32, 512, 8192, 30, "BAG"), (FP32, 512, 12_288, 30, "ANY"), (FP32, 512, 8192, 12, "ANY"),
+    (FP32, 256, 2048, 16, "ANY"), (INT8, 1024, 8191, 30, "BAG"), (INT8, 1024, 8192, 30, "ANY"),
+    (FP8, 1024, 1023, 9, "BAG"), (FP8, 1024, 1024, 100, "ANY"), (FP16, 512, 32_768, 8, "STREAM"),
+])
+def test_kernel_of_one_group(pkg, ty, D, bags, rows, want):
+    c = pkg.capi
+    assert kinds(pkg, [(1000, D, ty)], bags, rows) == [getattr(c, "TBE_POOLED_" + want)]
