@@ -883,7 +883,7 @@ __global__ __launch_bounds__(kBBBlock) void scan_tiles_based(const T* __restrict
 
 // A work-group has a wave per row (W of both), as the general path deals them: with 2 or 4
 // consecutive rows a wave, a feature of long rows was left to a few waves (96 features x 128
-// rows, 737 k int32 indices, 90 % of them in one feature: 224 us, the general path 77, now 95).
+// rows, 737 k int32 indices, 90 % of them in one feature: 224 us, the general path 77, now 76).
 
 template <typename IT, typename OT, int W>
 __global__ __launch_bounds__(W * kWaveBB) void bb_count_few(BBParams<IT, OT> p, const OT* __restrict__ lengths,
@@ -1004,24 +1004,28 @@ __global__ __launch_bounds__(W * kWaveBB) void bb_scatter_few(BBParams<IT, OT> p
 
 // Rows (and waves) per work-group of the two launches, 0 where the general path is used.
 // The lines (us as general / two launches; int64, rows of 30 indices unless said):
-//  * A work-group reads all lengths before its rows and all bucket totals: fewer, larger ones
-//    from 2048 and 4096 rows and past 8 k totals (3328 rows, 16 ranks: 8 rows a group 27 /
-//    17, 16 rows 21).  Past 32 ranks 16 waves share the totals' sums (1536 rows, 64 ranks:
-//    27 / 20; 4 rows a group 34).
-//  * 16 waves of int64 indices fill a CU's LDS, and all wait for the sums: 8192 rows, 8
-//    ranks 35 / 27, 12288 rows 42 / 40, but with 90 % of the indices in one of 96 features
-//    57 / 66.  int32 (two groups a CU): 12288 rows 38 / 31 and 53 / 58, 16384 rows 44 / 39
-//    and 50 / 55.
+//  * A work-group reads all lengths before its rows and all bucket totals, so fewer and
+//    larger ones from 2048 rows (of 8 ranks or more; 5220 rows, 4 ranks: 4 rows a group 25,
+//    8 rows 17, 16 rows 25) and past 8 k totals.  16 rows fill a CU's LDS and all wait for
+//    the sums (3328 rows, 16 ranks: 8 rows a group 17, 16 rows 21): only past 12 k totals,
+//    and past 32 ranks, whose sums 16 waves share (1536 rows, 64 ranks: 27 / 20, 4 rows 34).
+//  * Long rows side by side share a CU, those of a rank or two its counters as well: 4 rows
+//    (2560 rows of 100, 90 % in one of 32 features, 1 rank: 58 / 49, 8 rows 65).
+//  * 8192 rows, 8 ranks 35 / 26, 12288 rows 42 / 36 and with 90 % of the indices in one
+//    feature 57 / 56; in groups of 16 rows (16 ranks) 44 / 44 and 58 / 69: those up to 8192.
 //  * Past a million indices the general scatter's fast pass, of more waves per SIMD, is worth
 //    its launches (8192 rows, 16 ranks, 2.6 M indices 43.8 / 45.6).  Bucket boundaries keep
 //    rows from it: four million (12288 rows, 8 ranks, 737 k int32 49 / 39).
 constexpr int64_t kFewIndices = int64_t(1) << 20;
 
-int few_rows_per_group(int64_t my, int64_t L, int64_t N, bool lists, int32_t index_size) {
-  if (my > kWaveBB || L < 1 || N > (lists ? 4 : 1) * kFewIndices) return 0;
-  if (L > (lists || index_size == 4 ? 12288 : 8192)) return 0;
-  for (int per = my > 32 || L > 4096 ? 16 : L > 2048 ? 8 : 4; per <= 16; per *= 2)
-    if ((L + per - 1) / per * my <= (per < 16 ? 8192 : 16384)) return per;
+int few_rows_per_group(int64_t my, int64_t L, int64_t N, bool lists) {
+  if (my > kWaveBB || L < 1 || L > 12288 || N > (lists ? 4 : 1) * kFewIndices) return 0;
+  int per = 8;
+  if (my > 32) per = 16;
+  else if (L <= 2048 || (L <= 4096 && my < 8) || my == 1) per = 4;
+  const int most = lists || L <= 8192 ? 16 : 8;
+  for (; per <= most; per *= 2)
+    if ((L + per - 1) / per * my <= (per == 4 ? 8192 : per == 8 ? 12288 : 16384)) return per;
   return 0;
 }
 
@@ -1140,7 +1144,7 @@ int run(const TbeBlockBucketizeArgs* a, hipStream_t s, void* ws, int64_t sums_of
   p.keep = a->keep_orig_idx;
   int nbits = 0;  // ceil(log2(my_size))
   while (nbits < 6 && (int64_t(1) << nbits) < a->my_size) ++nbits;
-  const int per = few_rows_per_group(a->my_size, p.L, p.N, p.pos != nullptr, a->index_size);
+  const int per = few_rows_per_group(a->my_size, p.L, p.N, p.pos != nullptr);
   if (per > 0) {
     const int64_t groups = (p.L + per - 1) / per;
     if (groups * a->my_size * static_cast<int64_t>(sizeof(OT)) <= few_bytes) {
