@@ -1758,7 +1758,10 @@ __global__ __launch_bounds__(kBlock) void pooled_wide_kernel(KParams p) {
       case TBE_TY_INT4: pool_bag_wide<TBE_TY_INT4, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_INT8: pool_bag_wide<TBE_TY_INT8, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_INT2: pool_bag_wide<TBE_TY_INT2, WEIGHTED>(p, td, start, L, ct, b); break;
-      case TBE_TY_FP8:  pool_bag_wide<kTyFp8Wide,  WEIGHTED>(p, td, start, L, ct, b); break;
+      case TBE_TY_FP8:
+        if (p.fp8.h16_ok) pool_bag_wide<TBE_TY_FP8, WEIGHTED>(p, td, start, L, ct, b);
+        else pool_bag_wide<kTyFp8Wide, WEIGHTED>(p, td, start, L, ct, b);
+        break;
       case TBE_TY_FP16: pool_bag_wide<TBE_TY_FP16, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_BF16: pool_bag_wide<TBE_TY_BF16, WEIGHTED>(p, td, start, L, ct, b); break;
       case TBE_TY_FP32: pool_bag_wide<TBE_TY_FP32, WEIGHTED>(p, td, start, L, ct, b); break;

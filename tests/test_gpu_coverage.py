@@ -188,6 +188,35 @@ def test_table_past_2pow32_rows(pkg, oracle, gpu, pm, weighted):
         torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("eb,bias", [(4, 7), (5, 15)])
+def test_fp8_table_past_2pow32_rows(pkg, oracle, gpu, eb, bias):
+    """FP8 codes in the generic pooled kernel: read as fp16 (4 exponent bits), and decoded
+    by parts (5).  Rows past 2^32 of a table of 4-byte rows."""
+    from fbgemm_ascend_amd import IntNBitTableBatchedEmbeddingBagsCodegen, SparseType
+    if _free_gib() < 48:
+        pytest.skip("needs ~20 GiB of free HBM")
+    E, B = 2 ** 32 + 8, 40
+    m = IntNBitTableBatchedEmbeddingBagsCodegen([(E, 4, SparseType.FP8)], device=gpu, output_dtype=FP32,
+                                                indices_dtype=torch.int64, row_alignment=4, fp8_exponent_bits=eb,
+                                                fp8_exponent_bias=bias)
+    try:
+        g = torch.Generator(device=gpu)
+        g.manual_seed(eb)
+        w = m.weights_dev
+        for lo in (0, 4 * (E - 4000)):  # the rows read
+            w[lo:lo + 16000] = torch.randint(0, 256, (16000,), dtype=torch.uint8, device=gpu, generator=g)
+        L = torch.randint(0, 90, (B,), device=gpu, generator=g)
+        off = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), L.cumsum(0)])
+        idx = torch.randint(0, 4000, (int(off[-1]),), device=gpu, generator=g)
+        idx[::2] += E - 4000
+        for weighted in (False, True):
+            psw = torch.rand(idx.numel(), device=gpu, generator=g) if weighted else None
+            _check_module(oracle, m, idx, off, psw, f"FP8 {eb}/{bias} past 2^32 rows w={weighted}")
+    finally:
+        del m
+        torch.cuda.empty_cache()
+
+
 def test_more_than_2pow31_indices(pkg, gpu):
     """A call with 2^31 + 4096 indices (positions past 32 bits take the generic
     kernel).  Exact known answer: an FP32 D=4 table whose element c of row r is
