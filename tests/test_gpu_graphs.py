@@ -2,7 +2,7 @@
 permute_pooled_embs and block_bucketize_sparse_features; and the TBE forward called
 concurrently from several caller streams and host threads.
 
-A serving loop captures the lookup once and replays it; the TBE forward forks its
+A serving loop captures the lookup once and replays it; a large TBE forward forks its
 table groups onto library streams and joins them back with events, which must come
 along into the capture.  Each case warms the op up eagerly (plan cached, library
 streams created), captures one call, then replays the graph several times with new
@@ -20,7 +20,8 @@ FP32, FP16, INT8, INT4, INT2, BF16, FP8 = 0, 1, 2, 3, 4, 5, 6
 
 
 def _mixed_module(pkg, gpu, pm, out_ty, B=96, seed=11):
-    """Tables of four row types and widths: several table groups, so the group streams run."""
+    """Tables of four row types and widths: six table groups, one launch in small calls, a
+    launch per group on the group streams in large ones (test_gpu_group_routes.py)."""
     from fbgemm_ascend_amd import IntNBitTableBatchedEmbeddingBagsCodegen, SparseType
     specs = [(5000, 64, SparseType.INT4), (3000, 128, SparseType.INT8), (2000, 32, SparseType.FP16),
              (4000, 256, SparseType.INT2), (1000, 128, SparseType.INT4), (6000, 64, SparseType.FP8)]
@@ -46,9 +47,8 @@ def _inputs(m, gpu, B, seed, weighted):
 
 
 @pytest.mark.parametrize("pm,weighted,out_ty", [(0, False, FP16), (1, True, FP32), (2, False, BF16)])
-def test_tbe_forward_graph_replays(pkg, gpu, pm, weighted, out_ty):
+def test_tbe_forward_graph_replays(pkg, gpu, pm, weighted, out_ty, B=96):
     m = _mixed_module(pkg, gpu, pm, out_ty)
-    B = 96
     # inputs of equal sizes for every replay: same bag lengths, new rows and weights
     idx0, off0, psw0 = _inputs(m, gpu, B, 1, weighted)
     s = torch.cuda.Stream()
@@ -124,15 +124,15 @@ def test_permute_pooled_embs_graph_replays(pkg, gpu):
         assert torch.equal(y, want), f"replay {rep}"
 
 
-def test_concurrent_caller_streams_and_threads(pkg, gpu):
+def test_concurrent_caller_streams_and_threads(pkg, gpu, B=80):
     """Two modules of different layouts called alternately on two caller streams, and from
     two host threads: each caller stream gets its own library streams and each layout its
     own cached plan, so every output equals the same call made alone."""
     import threading
     ma = _mixed_module(pkg, gpu, 0, FP16, seed=21)
     mb = _mixed_module(pkg, gpu, 1, FP32, seed=22)
-    ia, oa, pa = _inputs(ma, gpu, 80, 3, False)
-    ib, ob, pb = _inputs(mb, gpu, 80, 4, True)
+    ia, oa, pa = _inputs(ma, gpu, B, 3, False)
+    ib, ob, pb = _inputs(mb, gpu, B, 4, True)
     want_a = ma(ia, oa, pa)
     want_b = mb(ib, ob, pb)
     torch.cuda.synchronize()
@@ -170,12 +170,12 @@ def test_concurrent_caller_streams_and_threads(pkg, gpu):
 
 
 @pytest.mark.parametrize("sequence,weighted", [(False, False), (True, True)])
-def test_block_bucketize_graph_replays(pkg, gpu, sequence, weighted):
-    """block_bucketize_sparse_features captured once (its offsets scan, count, scan and
-    scatter kernels) and replayed with new indices and weights of the same lengths."""
+def test_block_bucketize_graph_replays(pkg, gpu, sequence, weighted, case=None):
+    """block_bucketize_sparse_features captured once (1024 rows: its count and scatter
+    kernels) and replayed with new indices and weights of the same lengths."""
     import numpy as np
     from _bucketize_cases import CASES, gen_case
-    case = next(c for c in CASES if c.name == "i64_pow2_basic")
+    case = case or next(c for c in CASES if c.name == "i64_pow2_basic")
     lengths, indices, block_sizes, w = gen_case(case, 7, weights=weighted)[:4]
     L = torch.as_tensor(lengths, device=gpu)
     I = torch.as_tensor(indices, device=gpu)

@@ -267,8 +267,8 @@ def test_double_table_forward_nobag(pkg, oracle, gpu, tables, out_ty):
 
 def test_c_abi_matches_torch_op(pkg, gpu):
     """The C ABI called directly (ctypes) gives the torch op's exact output, with and
-    without the XCD block renumbering, and with the table groups on the caller's
-    stream instead of the two group streams."""
+    without the XCD block renumbering and the group streams (which the 16 k bags of
+    config 3 do not use: test_gpu_group_routes.py)."""
     from fbgemm_ascend_amd.workloads import make_workload
     for cid in (1, 3):
         wl = make_workload(cid, device=gpu, scale_rows=0.01, batch=256)

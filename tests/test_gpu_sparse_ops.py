@@ -183,8 +183,8 @@ def test_bucketize_indices_beyond_blocks(pkg, oracle, gpu, dtype, my_size, tnb):
 @pytest.mark.parametrize("at", [5, 600, 1500])
 def test_bucketize_high_index_in_one_chunk(pkg, oracle, gpu, dtype, my_size, at):
     # rows of 400-1800 indices, every third one with a single index at or above the
-    # blocks at position `at`: the fast scatter pass writes the chunks before it,
-    # gives the row up at that chunk, and the general pass rewrites the whole row
+    # blocks at position `at` (48 rows: the two launches; test_gpu_group_routes.py has the
+    # same for the general path's fast and general pass)
     from _bucketize_cases import Case
     case = Case(f"high_at{at}_my{my_size}", 4, 12, 400, 1800, 8, 40, my_size, dtype)
     for seed, kw in ((51, dict(weights=True, sequence=True)), (52, dict(sequence=True, keep=True)),
