@@ -1419,7 +1419,9 @@ __device__ __forceinline__ void decode_word(uint32_t d, float (&v)[Traits<WT>::k
 // loads of a chunk unrolled.  us, 26 tables, 1.6 M indices unless said, unrolled -> batches:
 // INT8 D 64 / 128 80 -> 73 / 160 -> 131, FP8 D 64 / 128 70 -> 56 / 189 -> 105, FP16 D 64
 // 106 -> 55, FP32 D 16 36 -> 31, INT4 D 256 / 512 (0.8 / 0.4 M indices) 124 -> 84 /
-// 120 -> 86.  The others lose or draw: INT8 D 256 57 -> 62, BF16 D 128 154 -> 159, INT4
+// 120 -> 86.  (fp16 out; fp32: FP16 D 64 106 -> 76, FP32 D 32 84 -> 47, INT4 D 256 (0.2 M) 97
+// -> 95, INT8 and FP8 bound by their stores: D 64 81 -> 80, D 128 143 and 147 either way.)
+// The others lose or draw: INT8 D 256 57 -> 62, BF16 D 128 154 -> 159, INT4
 // D 64 62 -> 64, INT2 D 256 170 -> 228.
 template <int WT, int LG>
 constexpr bool nobag_batches() {
